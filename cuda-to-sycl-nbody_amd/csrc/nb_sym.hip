@@ -64,6 +64,7 @@
 //
 // Build with -ffp-contract=off (explicit fmaf only).
 
+#include "nb_pair_block.hpp"
 #include "nb_pairs.hpp"
 
 #include <vector>
@@ -184,6 +185,17 @@ struct ForceRule : PlainPartials<3> {
   static constexpr bool MASKED_TAIL = false;
   // every sum rotates with lds_rol1 (see wave_rol1)
   static constexpr bool rotate_lds(int) { return true; }
+  // passes with reactions and without masks run the pair term as a block of
+  // assembly per source (nb_pair_block.hpp)
+  static constexpr bool BLOCK = true;
+
+  template <int U, bool PRIO>
+  static __device__ __forceinline__ void block(const float (&s)[SRC],
+                                               const float (&t)[U][SRC],
+                                               float (&a)[U][ACC],
+                                               float (&rs)[ACC], float eps) {
+    force_block<U, PRIO>(s, t, a, rs, eps);
+  }
 
   static __device__ __forceinline__ void load(const SymArgs &a, int j,
                                               float (&v)[SRC]) {
@@ -235,6 +247,7 @@ struct ForceRule : PlainPartials<3> {
 // sum is s - c).  A partial is (s_x, s_y, s_z, c_x, c_y, c_z); the finalize
 // Kahan-adds the partials' values s - c.
 struct KahanForceRule {
+  static constexpr bool BLOCK = false;
   static constexpr int SRC = 3;
   static constexpr int ACC = 6;
   static constexpr bool MASKED_TAIL = false;
@@ -310,6 +323,7 @@ struct KahanForceRule {
 
 template <bool FUSED>
 struct AdjointRule : PlainPartials<FUSED ? 6 : 3> {
+  static constexpr bool BLOCK = false;
   static constexpr int SRC = 6; // x, y, z, g_x, g_y, g_z
   static constexpr int ACC = FUSED ? 6 : 3; // sum M (g_j - g_k) [, F]
   static constexpr bool MASKED_TAIL = true;
@@ -479,6 +493,15 @@ __device__ __forceinline__ void tile_pass(Lane<R, U> &L, const float *src,
           sv[4 * qq + 3][c] = v.w;
         }
       }
+    }
+    if constexpr (R::BLOCK && SYM && !MASK) {
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        R::template block<U, PRIO>(sv[q], L.t, L.a, L.rs[q], eps);
+#pragma unroll
+        for (int c = 0; c < R::ACC; ++c) L.rs[q][c] = lds_rol1(L.rs[q][c]);
+      }
+      return;
     }
 #pragma unroll
     for (int q = 0; q < U; ++q) {
