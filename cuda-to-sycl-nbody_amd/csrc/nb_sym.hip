@@ -17,33 +17,36 @@
 // order in which each particle's terms are summed differs from the
 // target-sharded kernels.
 //
-// Decomposition (U particles per lane, P = 64 U per wave, ST = 4 P):
-//   * particles are grouped in super-tiles of ST; a work item is one
-//     workgroup (4 waves) and a chunk of one row of the super-tile pair
-//     triangle: super-tile GA against super-tiles GB in [GB0, GB1), GB >= GA;
-//   * wave w holds the inputs and sums of targets 4 GA + w (tile of P) in
-//     VGPRs; the source super-tile sits in LDS;
-//   * for GB > GA, in pass b wave w meets source tile j = (w + b) & 3; in
-//     each of 64 steps lane l takes the U sources of set (l + s) & 63 from
-//     LDS and evaluates the U x U pair terms, adding the (negated) reaction
-//     to U per-source sums that rotate one lane down the wave (wave_rol1 or
-//     lds_rol1) after each step, so that after 64 steps lane l again holds
-//     set l's sums.  Between passes the reaction sums of the four tiles live in LDS
-//     (each tile is owned by one wave per pass); after pass 3 the chunk
-//     writes them as the (GA, GB) reaction partial;
-//   * for GB == GA (first super-tile of a row) each wave meets its own tile
-//     without reactions (self terms are +0) and then, with 2 or 4 per lane,
-//     the tiles above it with reactions (each of the six tile pairs once),
-//     subtracting at the end the reactions its tile received; with 8 per
-//     lane it meets the other three tiles without reactions as well;
-//   * the targets' sums over the chunk are one row partial;
-//   * a finalize kernel sums, per particle, its row partials in chunk order
-//     and then subtracts the reaction partials of its column in GA order,
-//     and applies the rule's epilogue.  The order is fixed: results are
-//     deterministic.
-// Two more forms reuse the same passes: one tile pair per wave for small n
-// (sym_tile_kernel) and the super-tile pairs of many independent systems on
-// one persistent queue (sym_batch_kernel).
+// Particles are grouped in super-tiles of ST; a work item is one workgroup (4
+// waves) and a chunk of one row of the super-tile pair triangle: super-tile
+// GA against super-tiles GB in [GB0, GB1), GB >= GA.  Each item writes the
+// targets' sums over its chunk as one row partial and, per pair with GB > GA,
+// the (negated) reaction sums of GB's particles.  A finalize kernel sums, per
+// particle, its row partials in chunk order, then subtracts the reaction
+// partials of its column in GA order, and applies the rule's epilogue.  The
+// order is fixed: results are deterministic.
+// Two forms of the pair kernel:
+//   * row form (sym_row_kernel; ST = 128, 256, 512): a wave holds all
+//     targets of GA and meets GB in sets of 64 sources (see row_item).  The
+//     shapes with 2 particles per lane of the workgroup (ST = 512) and the
+//     tile pairs;
+//   * four-wave form (sym_kernel; U = 4 or 8 per lane, P = 64 U per wave, ST =
+//     4 P): wave w holds targets 4 GA + w (tile of P) in VGPRs; the source
+//     super-tile sits in LDS; for GB > GA, in pass b wave w meets source tile
+//     j = (w + b) & 3; in each of 64 steps lane l takes the U sources of set
+//     (l + s) & 63 from LDS and evaluates the U x U pair terms, adding the
+//     (negated) reaction to U per-source sums that rotate one lane down the
+//     wave (wave_rol1 or lds_rol1) after each step, so that after 64 steps
+//     lane l again holds set l's sums.  Between passes the reaction sums of
+//     the four tiles live in LDS (each tile is owned by one wave per pass).
+//     For GB == GA each wave meets its own tile without reactions (self terms
+//     are +0) and then, with 4 per lane, the tiles above it with reactions
+//     (each of the six tile pairs once), subtracting at the end the reactions
+//     its tile received; with 8 per lane it meets the other three tiles
+//     without reactions as well.  A quarter of the row form's reaction
+//     partials per pair: the choice where those dominate (n >= 2^18).
+// The super-tile pairs of many independent systems also run on one
+// persistent queue (sym_batch_kernel, sym_row_batch_kernel).
 // Padding (index >= n): ForceRule puts padding particles at 1e30 in every
 // coordinate, so any pair with a real particle has |r|^2 = +inf,
 // rsqrt(inf) = 0 and r * 0 = 0 (exact zeros, no mask; a pair of two padding
@@ -57,10 +60,11 @@
 //
 // Per pair term (two interactions): forward 14 VALU + v_rsq_f32 + 3/U
 // reaction moves through the LDS crossbar (ds_bpermute, no VALU slot);
-// adjoint 25 VALU + v_rsq_f32 (K and 1/d from rsqrt(d)) + 3/U DPP moves;
-// fused adjoint 33 VALU + v_rsq_f32 (K as the forward rule forms it, 1/d =
-// K^2 d^2) + 6/U DPP moves.  The target-sharded kernels spend 11 (forward)
-// and 22 (adjoint) VALU per interaction.
+// adjoint 25 VALU + v_rsq_f32 (K and 1/d from rsqrt(d)) + 3/U moves; fused
+// adjoint 33 VALU + v_rsq_f32 (K as the forward rule forms it, 1/d = K^2 d^2)
+// + 6/U moves; Kahan sums 32 VALU + v_rsq_f32 + 6/U moves.  The
+// target-sharded kernels spend 11 (forward) and 22 (adjoint) VALU per
+// interaction.
 //
 // Build with -ffp-contract=off (explicit fmaf only).
 
@@ -73,8 +77,6 @@ namespace nb {
 namespace {
 
 constexpr int kWaves = 4;        // waves per workgroup = tiles per super-tile
-constexpr size_t kTilePrioMaxParticles = 32768; // see launch_forward_sym
-constexpr size_t kKahanTilePrioMaxParticles = 16384; // the same, Kahan sums
 constexpr float kFar = 1.0e30f;  // coordinate of ForceRule padding particles
 constexpr int kDppWaveRol1 = 0x134;
 
@@ -89,13 +91,11 @@ constexpr int kDppWaveRol1 = 0x134;
 //              cycles, measured with probe/issue_rates.hip), while the
 //              permute's latency is hidden (each sum is rotated as soon as
 //              it is complete and read again only in the next step).  The
-//              forward rules rotate with lds_rol1 (N = 262144: 11.3 vs 11.9
-//              ms with plain sums, 22.5 vs 23.8 ms with Kahan sums; the
-//              64-system batch 4.43 vs 4.52 ms); the adjoint rules, whose
-//              loops read twice the LDS per step already, keep DPP for the
-//              adjoint sums (lds_rol1 for all of them measured 1.5 % slower
-//              for the adjoint, 4 % for the fused step) and the fused step
-//              rotates its force sums with lds_rol1.
+//              row form and the forward rules rotate with lds_rol1; the
+//              adjoint rules' four-wave form, whose loop reads twice the LDS
+//              per step already, keeps DPP for the adjoint sums (lds_rol1
+//              for all of them measured 1.5 % slower for the adjoint, 4 % for
+//              the fused step).
 __device__ __forceinline__ float wave_rol1(float v) {
   const int b = __builtin_bit_cast(int, v);
   return __builtin_bit_cast(
@@ -185,16 +185,17 @@ struct ForceRule : PlainPartials<3> {
   static constexpr bool MASKED_TAIL = false;
   // every sum rotates with lds_rol1 (see wave_rol1)
   static constexpr bool rotate_lds(int) { return true; }
-  // passes with reactions and without masks run the pair term as a block of
-  // assembly per source (nb_pair_block.hpp)
+  // the four-wave super-tile passes run the pair term as a block of assembly
+  // per source (nb_pair_block.hpp); the row form does for every rule
   static constexpr bool BLOCK = true;
+  static constexpr bool WAVE8 = true; // four-wave kernels with 8 per lane
 
-  template <int U, bool PRIO>
+  template <int U>
   static __device__ __forceinline__ void block(const float (&s)[SRC],
                                                const float (&t)[U][SRC],
                                                float (&a)[U][ACC],
                                                float (&rs)[ACC], float eps) {
-    force_block<U, PRIO>(s, t, a, rs, eps);
+    force_block<U>(s, t, a, rs, eps);
   }
 
   static __device__ __forceinline__ void load(const SymArgs &a, int j,
@@ -248,8 +249,18 @@ struct ForceRule : PlainPartials<3> {
 // Kahan-adds the partials' values s - c.
 struct KahanForceRule {
   static constexpr bool BLOCK = false;
+  static constexpr bool WAVE8 = false;
   static constexpr int SRC = 3;
   static constexpr int ACC = 6;
+
+  template <int U>
+  static __device__ __forceinline__ void block(const float (&s)[SRC],
+                                               const float (&t)[U][SRC],
+                                               float (&a)[U][ACC],
+                                               float (&rs)[ACC], float eps) {
+    kahan_block<U>(s, t, a, rs, eps);
+  }
+
   static constexpr bool MASKED_TAIL = false;
   // every sum rotates with lds_rol1 (see wave_rol1)
   static constexpr bool rotate_lds(int) { return true; }
@@ -324,12 +335,22 @@ struct KahanForceRule {
 template <bool FUSED>
 struct AdjointRule : PlainPartials<FUSED ? 6 : 3> {
   static constexpr bool BLOCK = false;
+  static constexpr bool WAVE8 = true;
   static constexpr int SRC = 6; // x, y, z, g_x, g_y, g_z
   static constexpr int ACC = FUSED ? 6 : 3; // sum M (g_j - g_k) [, F]
   static constexpr bool MASKED_TAIL = true;
-  // the adjoint sums rotate by DPP; the fused step's force sums (3..5) with
-  // lds_rol1 (N = 262144: 24.4 vs 25.1 ms; all six through the crossbar: 26.1
-  // ms; any of the plain adjoint's through it: no gain)
+
+  template <int U>
+  static __device__ __forceinline__ void block(const float (&s)[SRC],
+                                               const float (&t)[U][SRC],
+                                               float (&a)[U][ACC],
+                                               float (&rs)[ACC], float eps) {
+    if constexpr (FUSED) fused_block<U>(s, t, a, rs, eps);
+    else adjoint_block<U>(s, t, a, rs, eps);
+  }
+
+  // four-wave form: the adjoint sums rotate by DPP, the fused step's force
+  // sums (3..5) with lds_rol1
   static constexpr bool rotate_lds(int c) { return FUSED && c >= 3; }
 
   // g = lv' + dt lx' (the cotangent the pair sum is taken of)
@@ -427,13 +448,11 @@ struct AdjointRule : PlainPartials<FUSED ? 6 : 3> {
 // holds members 4 qq .. 4 qq + 3 of set m, so the 64 lanes of a step (sets
 // (l + s) mod 64, one quad each) read one contiguous 1 KiB block: no bank
 // conflicts.
-// With U = 2 (tile-pair form only) set m's two members sit in float2 slot m.
 template <int U>
 __device__ __forceinline__ int lds_slot(int o) {
   constexpr int P = 64 * U;
   const int j = o / P, r = o % P;
   const int m = r / U, q = r % U;
-  if constexpr (U == 2) return j * P + m * 2 + q;
   return j * P + (q >> 2) * 256 + m * 4 + (q & 3);
 }
 
@@ -451,53 +470,35 @@ struct Lane {
 // target validity; sources are valid below index n).  With SELF (a wave's
 // pass over its own tile, with MASK) the self pairs contribute nothing
 // either: needed when eps^3 is not a normal float.
-// [s0, s1): the steps of the pass this call runs (a half pass leaves lane l
-// with the reaction sums of set (l + s1) mod 64).
-// PRIO: the wave lowers its issue priority at each quarter of the pass
-// (s_setprio 3, 2, 1, 0), so that the SIMD's arbiter, which otherwise
-// favours the oldest wave, lets the waves that lag behind catch up.  Used by
-// the tile-pair forms (forward up to n = 32768, Kahan sums up to 16384,
-// adjoint and two-item forms at every size they run), where most waves of the launch start at once
-// and, without it, finish between 10 and 37 us into a 40 us kernel (n =
-// 12800, per-wave clock stamps): the last quarter of the launch ran on one
-// or two waves per SIMD.
-template <class R, int U, bool SYM, bool MASK, bool SELF = false,
-          bool PRIO = false>
+template <class R, int U, bool SYM, bool MASK, bool SELF = false>
 __device__ __forceinline__ void tile_pass(Lane<R, U> &L, const float *src,
                                           int j, int lane, float eps,
                                           const bool (&vt)[U], int src0,
-                                          int n, int s0 = 0, int s1 = 64) {
+                                          int n) {
   static_assert(!SELF || (MASK && !SYM), "self pairs: masked own-tile pass");
   constexpr int P = 64 * U;
   constexpr int ST = kWaves * P;
   constexpr int Q = U / 4;
-  static_assert(U == 2 || U % 4 == 0, "particles per lane: 2 or a multiple of 4");
+  static_assert(U % 4 == 0, "particles per lane: a multiple of 4");
   auto step = [&](int s) {
     const int m = (lane + s) & 63;
     float sv[U][R::SRC];
 #pragma unroll
     for (int c = 0; c < R::SRC; ++c) {
-      if constexpr (U == 2) {
-        const float2 v = reinterpret_cast<const float2 *>(src + c * ST + j * P)[m];
-        sv[0][c] = v.x;
-        sv[1][c] = v.y;
-      } else {
-        const float4 *p4 =
-            reinterpret_cast<const float4 *>(src + c * ST + j * P);
+      const float4 *p4 = reinterpret_cast<const float4 *>(src + c * ST + j * P);
 #pragma unroll
-        for (int qq = 0; qq < Q; ++qq) {
-          const float4 v = p4[qq * 64 + m];
-          sv[4 * qq + 0][c] = v.x;
-          sv[4 * qq + 1][c] = v.y;
-          sv[4 * qq + 2][c] = v.z;
-          sv[4 * qq + 3][c] = v.w;
-        }
+      for (int qq = 0; qq < Q; ++qq) {
+        const float4 v = p4[qq * 64 + m];
+        sv[4 * qq + 0][c] = v.x;
+        sv[4 * qq + 1][c] = v.y;
+        sv[4 * qq + 2][c] = v.z;
+        sv[4 * qq + 3][c] = v.w;
       }
     }
     if constexpr (R::BLOCK && SYM && !MASK) {
 #pragma unroll
       for (int q = 0; q < U; ++q) {
-        R::template block<U, PRIO>(sv[q], L.t, L.a, L.rs[q], eps);
+        R::template block<U>(sv[q], L.t, L.a, L.rs[q], eps);
 #pragma unroll
         for (int c = 0; c < R::ACC; ++c) L.rs[q][c] = lds_rol1(L.rs[q][c]);
       }
@@ -524,20 +525,7 @@ __device__ __forceinline__ void tile_pass(Lane<R, U> &L, const float *src,
               R::rotate_lds(c) ? lds_rol1(L.rs[q][c]) : wave_rol1(L.rs[q][c]);
     }
   };
-  if constexpr (PRIO) {
-    // the priority is set once per quarter, outside the step loop
-    const int qlen = (s1 - s0) >> 2; // 16 or 8 steps
-    for (int quarter = 0; quarter < 4; ++quarter) {
-      if (quarter == 0) __builtin_amdgcn_s_setprio(3);
-      else if (quarter == 1) __builtin_amdgcn_s_setprio(2);
-      else if (quarter == 2) __builtin_amdgcn_s_setprio(1);
-      else __builtin_amdgcn_s_setprio(0);
-      const int e = s0 + (quarter + 1) * qlen;
-      for (int s = s0 + quarter * qlen; s < e; ++s) step(s);
-    }
-  } else {
-    for (int s = s0; s < s1; ++s) step(s);
-  }
+  for (int s = 0; s < 64; ++s) step(s);
 }
 
 template <class R, int U, bool MASK>
@@ -795,7 +783,231 @@ __device__ __forceinline__ bool combine_runs(float (&f)[R::ACC],
   }
 }
 
-constexpr int kTileRuns = 4; // runs per particle, tile-pair finalize
+// ---- row form: one wave holds a whole row super-tile ------------------------
+//
+// Super-tiles of ST = 64 U particles, U targets per lane: each wave of the
+// workgroup holds all targets of the row super-tile GA and takes its share of
+// the source super-tile GB in sets of 64 sources, one source per lane and
+// step.  Per step a lane reads one source (SRC floats) from LDS and rotates
+// ACC reaction sums for U pair terms; no barrier inside a super-tile pair.
+//   * U >= 4: wave w meets sets w, w + 4, .. of GB (U / 4 of them) and writes
+//     their reaction sums;  U = 2: two waves share a set, each half of its 64
+//     steps, and add their reaction sums through LDS;
+//   * at the end of the work item the four waves' target sums are added in a
+//     fixed tree, (0 + 2) + (1 + 3), and written as one row partial.
+// Partials and finalize are those of the four-wave form with the same ST.
+// The sources lie twice in LDS (128 floats per coordinate and wave), so that
+// step s reads at lane + s with no wrap, its offset in the instruction.
+//
+// Why: with 2 targets x 2 sources per lane a step spends 6 permutes and 3
+// LDS reads on 4 pair terms (forward; 12 and 3 with Kahan sums, 6 .. 12 and 6
+// for the adjoint); with 8 x 1 it is 3 and 3 for 8.  In the pair loop alone,
+// sustained at 4 waves per SIMD, SIMD cycles (at 2.4 GHz) per wave pair term
+// 2 x 2 -> 8 x 1: forward 56 -> 47, adjoint 85 -> 72, fused 120 -> 94, Kahan
+// 102 -> 89.
+template <class R, int U>
+struct RowShape {
+  static_assert(U == 2 || U == 4 || U == 8, "targets per lane");
+  static constexpr int ST = 64 * U;                  // super-tile
+  static constexpr int PARTS = U >= 4 ? 1 : 4 / U;   // waves per set
+  static constexpr int STEPS = 64 / PARTS;           // steps of a wave per set
+  static constexpr int SRC_FLOATS = kWaves * R::SRC * 128;
+  static constexpr int REACT_FLOATS = PARTS > 1 ? kWaves * R::ACC * 64 : 0;
+  static constexpr int SUM_FLOATS = 2 * R::ACC * ST; // the tree's two buffers
+  static constexpr int LDS_FLOATS = SRC_FLOATS + REACT_FLOATS > SUM_FLOATS
+                                        ? SRC_FLOATS + REACT_FLOATS
+                                        : SUM_FLOATS;
+};
+
+// Orders the wave's own LDS writes before its later reads (other lanes read
+// them): the hardware runs a wave's LDS operations in order, the fences keep
+// the compiler from reordering them.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Steps [s0, s0 + STEPS) of the wave's targets t against the 64 sources at
+// src ([SRC][128]): target sums into a, reaction sums of source (lane + s1)
+// mod 64 into rs.  masked: sources at or past index n - src0 and, in the set
+// of the wave's own targets self (-1: another set), the self pairs (step 0)
+// contribute nothing.
+template <class R, int U>
+__device__ __forceinline__ void
+row_pass(const float (&t)[U][R::SRC], float (&a)[U][R::ACC],
+         float (&rs)[R::ACC], const float *src, int lane, int s0, float eps,
+         bool masked, int self, int valid) {
+  constexpr int STEPS = RowShape<R, U>::STEPS;
+  const float *p = src + lane + s0;
+  if (!masked) {
+#pragma unroll 4
+    for (int s = 0; s < STEPS; ++s) {
+      float sv[R::SRC];
+#pragma unroll
+      for (int e = 0; e < R::SRC; ++e) sv[e] = p[e * 128 + s];
+      R::template block<U>(sv, t, a, rs, eps);
+#pragma unroll
+      for (int e = 0; e < R::ACC; ++e) rs[e] = lds_rol1(rs[e]);
+    }
+  } else {
+#pragma unroll 1
+    for (int s = 0; s < STEPS; ++s) {
+      float sv[R::SRC];
+#pragma unroll
+      for (int e = 0; e < R::SRC; ++e) sv[e] = p[e * 128 + s];
+      const bool vs = ((lane + s0 + s) & 63) < valid;
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        R::template pair<true, true>(sv, t[k], a[k], rs, eps,
+                                     vs && !(k == self && s0 + s == 0));
+#pragma unroll
+      for (int e = 0; e < R::ACC; ++e) rs[e] = lds_rol1(rs[e]);
+    }
+  }
+}
+
+// Work item: row super-tile ga against source super-tiles [gb0, gb1), gb0 >=
+// ga.  Row partial ([ACC][ST]) to fp, the (negated) reaction sums of gb > ga
+// to sp_at(gb) ([ACC][ST]).  lds: LDS_FLOATS.  Called by every thread of the
+// workgroup.  The diagonal (gb == ga) is met whole, without reactions.
+template <class R, int U, class SpAt>
+__device__ __forceinline__ void row_item(const SymArgs &a, float *lds, int ga,
+                                         int gb0, int gb1, float *fp,
+                                         SpAt sp_at) {
+  using S = RowShape<R, U>;
+  constexpr int ST = S::ST;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int part = w % S::PARTS, first = w / S::PARTS;
+  const int s0 = part * S::STEPS;
+  float t[U][R::SRC], sum[U][R::ACC];
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    R::load(a, ga * ST + k * 64 + lane, t[k]);
+#pragma unroll
+    for (int e = 0; e < R::ACC; ++e) sum[k][e] = 0.0f;
+  }
+  float *src = lds + w * (R::SRC * 128);
+  float *react = lds + S::SRC_FLOATS;
+  const bool self_vanishes = self_term_vanishes(a.c.eps);
+  float nxt[R::SRC]; // the next set's sources, in flight during a pass
+  R::load(a, gb0 * ST + first * 64 + lane, nxt);
+  int gb = gb0, q = first;
+  while (gb < gb1) {
+    wave_lds_fence();
+#pragma unroll
+    for (int e = 0; e < R::SRC; ++e) {
+      src[e * 128 + lane] = nxt[e];
+      src[e * 128 + 64 + lane] = nxt[e];
+    }
+    wave_lds_fence();
+    const int g = gb, set = q;
+    q += kWaves;
+    if (q >= U) {
+      q = first;
+      ++gb;
+    }
+    if (gb < gb1) R::load(a, gb * ST + q * 64 + lane, nxt);
+
+    const int left = a.n - (g * ST + set * 64); // sources before the padding
+    bool masked = g == ga && !self_vanishes;
+    if constexpr (R::MASKED_TAIL) masked = masked || left < 64;
+    float rs[R::ACC];
+#pragma unroll
+    for (int e = 0; e < R::ACC; ++e) rs[e] = 0.0f;
+    if (left > 0) // the same for the waves that share a set
+      row_pass<R, U>(t, sum, rs, src, lane, s0, a.c.eps, masked,
+                     g == ga ? set : -1, left);
+    if (g == ga) continue;
+    float *sp = sp_at(g) + set * 64;
+    if constexpr (S::PARTS == 1) {
+#pragma unroll
+      for (int e = 0; e < R::ACC; ++e) sp[e * ST + lane] = rs[e];
+    } else {
+      // lane l holds the sums of source (l + s1) mod 64
+      const int m = (lane + s0 + S::STEPS) & 63;
+#pragma unroll
+      for (int e = 0; e < R::ACC; ++e) react[(w * R::ACC + e) * 64 + m] = rs[e];
+      __syncthreads();
+      if (part == 0) {
+        float f[R::ACC];
+        R::fetch(f, react + w * R::ACC * 64 + lane, 64);
+#pragma unroll
+        for (int p = 1; p < S::PARTS; ++p) {
+          float v[R::ACC];
+          R::fetch(v, react + (w + p) * R::ACC * 64 + lane, 64);
+          R::add_v(f, v);
+        }
+#pragma unroll
+        for (int e = 0; e < R::ACC; ++e) sp[e * ST + lane] = f[e];
+      }
+      __syncthreads(); // read before the next pair overwrites it
+    }
+  }
+
+  // target sums of the four waves: (0 + 2) + (1 + 3); waves 0 and 1 each
+  // finish half of the targets
+  auto put = [&](int slot, int k0, int k1) {
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+      if (k >= k0 && k < k1)
+#pragma unroll
+        for (int e = 0; e < R::ACC; ++e)
+          lds[(slot * R::ACC + e) * ST + k * 64 + lane] = sum[k][e];
+  };
+  auto take = [&](int slot, int k0, int k1) {
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+      if (k >= k0 && k < k1) {
+        float v[R::ACC];
+        R::fetch(v, lds + slot * (R::ACC * ST) + k * 64 + lane, ST);
+        R::add_v(sum[k], v);
+      }
+  };
+  __syncthreads(); // every wave is done with its sources
+  if (w >= 2) put(w - 2, 0, U);
+  __syncthreads();
+  if (w < 2) take(w, 0, U);
+  __syncthreads();
+  if (w == 0) put(0, U / 2, U);
+  if (w == 1) put(1, 0, U / 2);
+  __syncthreads();
+  if (w >= 2) return;
+  if (w == 0) take(1, 0, U / 2);
+  else take(0, U / 2, U);
+#pragma unroll
+  for (int k = 0; k < U; ++k)
+    if ((k < U / 2) == (w == 0))
+#pragma unroll
+      for (int e = 0; e < R::ACC; ++e)
+        fp[e * ST + k * 64 + lane] = sum[k][e];
+}
+
+// Work item -> (row ga, chunk c): rows are enumerated in order, row ga
+// holding ceil((ts - ga) / L) items.
+__device__ __forceinline__ int item_row(long long it, int ts, int L) {
+  int lo = 0, hi = ts - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (row_first(mid, ts, L) <= it) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
+template <class R, int U>
+__global__ __launch_bounds__(256) void sym_row_kernel(SymArgs a) {
+  __shared__ float lds[RowShape<R, U>::LDS_FLOATS];
+  constexpr int ST = RowShape<R, U>::ST;
+  const int ts = a.ts, L = a.chunk;
+  const long long it = blockIdx.x;
+  const int ga = item_row(it, ts, L);
+  const int gb0 = ga + (int)(it - row_first(ga, ts, L)) * L;
+  row_item<R, U>(a, lds, ga, gb0, min(gb0 + L, ts),
+                 a.fpart + (size_t)it * (R::ACC * ST), [&](int gb) {
+                   return a.spart + (size_t)pair_slot(ga, gb, ts) * (R::ACC * ST);
+                 });
+}
 
 template <class R, int U>
 __global__ __launch_bounds__(256) void sym_kernel(SymArgs a) {
@@ -807,17 +1019,8 @@ __global__ __launch_bounds__(256) void sym_kernel(SymArgs a) {
   float *sacc = reinterpret_cast<float *>(sacc4);
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int ts = a.ts, L = a.chunk;
-
-  // Work item -> (row ga, chunk c): rows are enumerated in order, row ga
-  // holding ceil((ts - ga) / L) items.
   const long long it = blockIdx.x;
-  int lo = 0, hi = ts - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (row_first(mid, ts, L) <= it) lo = mid;
-    else hi = mid - 1;
-  }
-  const int ga = lo;
+  const int ga = item_row(it, ts, L);
   const int c = (int)(it - row_first(ga, ts, L));
   const int gb0 = ga + c * L;
   const int gb1 = min(gb0 + L, ts);
@@ -832,25 +1035,34 @@ __global__ __launch_bounds__(256) void sym_kernel(SymArgs a) {
   store_row(T, a.fpart + (size_t)it * (R::ACC * ST), w, lane);
 }
 
+constexpr int kTileRuns = 4; // runs per particle, tile-pair finalize
+
 // Per particle: row partials (chunk order), minus the negated reaction
-// partials of its column (ga order); then the rule's epilogue.
-template <class R, int U>
+// partials of its column (ga order), in RUNS runs; then the rule's epilogue.
+template <class R, int ST, int RUNS>
 __global__ __launch_bounds__(256) void sym_finalize(SymArgs a) {
-  constexpr int ST = kWaves * 64 * U;
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= a.n) return;
-  const int g = i / ST, o = i % ST;
-  const int ts = a.ts, L = a.chunk;
-  const long long first = row_first(g, ts, L);
+  constexpr int PW = 256 / RUNS; // particles per workgroup
+  __shared__ float red[RUNS > 1 ? R::ACC : 1][256];
+  const int i = blockIdx.x * PW + threadIdx.x % PW;
+  const bool live = i < a.n;
+  if (RUNS == 1 && !live) return;
   float f[R::ACC];
-  run_sum<R, 1>(
-      f, (ts - g + L - 1) / L, g, 0,
-      [&](int c) { return a.fpart + (size_t)(first + c) * (R::ACC * ST) + o; },
-      [&](int ga) {
-        return a.spart + (size_t)pair_slot(ga, g, ts) * (R::ACC * ST) + o;
-      },
-      ST);
-  R::finish(a, i, f);
+  if (live) {
+    const int g = i / ST, o = i % ST;
+    const int ts = a.ts, L = a.chunk;
+    const long long first = row_first(g, ts, L);
+    run_sum<R, RUNS>(
+        f, (ts - g + L - 1) / L, g, threadIdx.x / PW,
+        [&](int c) { return a.fpart + (size_t)(first + c) * (R::ACC * ST) + o; },
+        [&](int ga) {
+          return a.spart + (size_t)pair_slot(ga, g, ts) * (R::ACC * ST) + o;
+        },
+        ST);
+  } else {
+#pragma unroll
+    for (int e = 0; e < R::ACC; ++e) f[e] = 0.0f;
+  }
+  if (combine_runs<R, RUNS>(f, red) && live) R::finish(a, i, f);
 }
 
 // ---- banded launches (n past the single-launch limit) ----------------------
@@ -880,6 +1092,22 @@ __host__ __device__ inline long long band_reactions(int b0, int w) {
   return (long long)b0 * w + (long long)w * (w - 1) / 2;
 }
 
+// Work item of a band -> row ga and first source super-tile gb0.
+__device__ __forceinline__ void band_item(long long it, int b0, int W, int L,
+                                          int &ga, int &gb0) {
+  const int c0 = (W + L - 1) / L; // items of a row above the band
+  const long long head = (long long)b0 * c0;
+  if (it < head) {
+    ga = (int)(it / c0);
+    gb0 = b0 + (int)(it % c0) * L;
+  } else { // the band's own triangle, rows enumerated in order
+    const long long j = it - head;
+    const int lo = item_row(j, W, L);
+    ga = b0 + lo;
+    gb0 = ga + (int)(j - row_first(lo, W, L)) * L;
+  }
+}
+
 template <class R, int U>
 __global__ __launch_bounds__(256) void sym_band_kernel(SymArgs a) {
   constexpr int P = 64 * U;
@@ -889,26 +1117,11 @@ __global__ __launch_bounds__(256) void sym_band_kernel(SymArgs a) {
   float *src = reinterpret_cast<float *>(src4);
   float *sacc = reinterpret_cast<float *>(sacc4);
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int L = a.chunk, b0 = a.b0, W = a.bw, b1 = b0 + W;
-  const int c0 = (W + L - 1) / L; // items of a row above the band
-  const long long head = (long long)b0 * c0;
+  const int L = a.chunk, b0 = a.b0, W = a.bw;
   const long long it = blockIdx.x;
   int ga, gb0;
-  if (it < head) {
-    ga = (int)(it / c0);
-    gb0 = b0 + (int)(it % c0) * L;
-  } else { // the band's own triangle, rows enumerated in order
-    const long long j = it - head;
-    int lo = 0, hi = W - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (row_first(mid, W, L) <= j) lo = mid;
-      else hi = mid - 1;
-    }
-    ga = b0 + lo;
-    gb0 = ga + (int)(j - row_first(lo, W, L)) * L;
-  }
-  const int gb1 = min(gb0 + L, b1);
+  band_item(it, b0, W, L, ga, gb0);
+  const int gb1 = min(gb0 + L, b0 + W);
   Lane<R, U> T;
   bool vt[U];
   load_targets(T, vt, a, ga, w, lane);
@@ -920,12 +1133,27 @@ __global__ __launch_bounds__(256) void sym_band_kernel(SymArgs a) {
   store_row(T, a.fpart + (size_t)it * (R::ACC * ST), w, lane);
 }
 
+// The same in the row form (U targets per lane, ST = 64 U).
+template <class R, int U>
+__global__ __launch_bounds__(256) void sym_row_band_kernel(SymArgs a) {
+  __shared__ float lds[RowShape<R, U>::LDS_FLOATS];
+  constexpr int ST = RowShape<R, U>::ST;
+  const int L = a.chunk, b0 = a.b0, W = a.bw;
+  const long long it = blockIdx.x;
+  int ga, gb0;
+  band_item(it, b0, W, L, ga, gb0);
+  row_item<R, U>(a, lds, ga, gb0, min(gb0 + L, b0 + W),
+                 a.fpart + (size_t)it * (R::ACC * ST), [&](int gb) {
+                   return a.spart + (size_t)band_pair_slot(ga, gb, b0, W) *
+                                        (R::ACC * ST);
+                 });
+}
+
 // Per particle: its band rows (chunk order) minus its band reactions (GA
 // order), added to the running sum (band order; Kahan sums carry their
 // compensation from band to band).
-template <class R, int U>
+template <class R, int ST>
 __global__ __launch_bounds__(256) void sym_band_fold(SymArgs a) {
-  constexpr int ST = kWaves * 64 * U;
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= a.n) return;
   const int g = i / ST, o = i % ST;
@@ -961,7 +1189,7 @@ __global__ __launch_bounds__(256) void sym_band_fold(SymArgs a) {
   for (int e = 0; e < R::ACC; ++e) acc[(size_t)e * a.n] = f[e];
 }
 
-template <class R, int U>
+template <class R>
 __global__ __launch_bounds__(256) void sym_band_finish(SymArgs a) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= a.n) return;
@@ -969,143 +1197,6 @@ __global__ __launch_bounds__(256) void sym_band_finish(SymArgs a) {
 #pragma unroll
   for (int e = 0; e < R::ACC; ++e) f[e] = a.acc3[(size_t)e * a.n + i];
   R::finish(a, i, f);
-}
-
-// ---- tile-pair items (small n) ----------------------------------------------
-//
-// Work item = one tile pair (A, B), A <= B, of P = 64 U particles, owned by
-// one wave; a workgroup holds four independent waves (one LDS tile each) and
-// has a single barrier, after staging.  The wave keeps the reaction sums in
-// registers for the whole pair.  Slot tri_slot(A, B, T) holds the row
-// partial [ACC][P] and, for A < B, the negated reaction partial [ACC][P].
-// T (T + 1) / 2 wave items fill the chip at sizes where the super-tile items
-// (T / 4)^2 / 2 workgroups of four waves) do not.
-
-// HALVES = 2 splits each tile pair into two work items of 32 steps (the
-// first and second half of the pass; item = 2 x pair + half), each with its
-// own row and reaction partial: twice the items, so that at small n the
-// launch holds more items than resident waves and the dispatcher keeps every
-// SIMD fed until a short tail, for twice the partials in the finalize.
-template <class R, int U, bool PRIO = false, int HALVES = 1>
-__global__ __launch_bounds__(256) void sym_tile_kernel(SymArgs a) {
-  static_assert(HALVES == 1 || HALVES == 2, "one or two items per tile pair");
-  constexpr int P = 64 * U;
-  constexpr int ST = kWaves * P;
-  __shared__ float4 src4[R::SRC][ST / 4]; // wave w's source tile is tile w
-  float *src = reinterpret_cast<float *>(src4);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int n = a.n, T = a.ts;
-  const long long items = (long long)HALVES * T * (T + 1) / 2;
-  const long long item = (long long)blockIdx.x * kWaves + w;
-  const bool live = item < items;
-  const long long pair = item / HALVES;
-  const int s0 = (int)(item % HALVES) * (64 / HALVES), s1 = s0 + 64 / HALVES;
-  int A = 0, B = 0;
-  if (live) { // row A: the last row whose first slot is <= pair
-    int lo = 0, hi = T - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (tri_slot(mid, mid, T) <= pair) lo = mid;
-      else hi = mid - 1;
-    }
-    A = lo;
-    B = A + (int)(pair - tri_slot(A, A, T));
-  }
-  // targets first: their loads are in flight while the source tile is staged
-  Lane<R, U> L;
-  bool vt[U];
-  const int t0 = A * P + lane * U;
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    R::load(a, t0 + k, L.t[k]);
-    vt[k] = t0 + k < n;
-#pragma unroll
-    for (int e = 0; e < R::ACC; ++e) L.a[k][e] = 0.0f;
-  }
-#pragma unroll
-  for (int r = 0; r < U; ++r) {
-    const int o = r * 64 + lane;
-    float v[R::SRC];
-    R::load(a, B * P + o, v);
-    const int d = lds_slot<U>(w * P + o);
-#pragma unroll
-    for (int e = 0; e < R::SRC; ++e) src[e * ST + d] = v[e];
-  }
-  __syncthreads(); // the only barrier: every wave has staged its tile
-  if (!live) return;
-  float *slot = a.fpart + (size_t)item * (2 * R::ACC * P);
-  bool masked = false;
-  if constexpr (R::MASKED_TAIL) masked = (n % P) != 0 && B == T - 1;
-  if (A == B) {
-    if (!self_term_vanishes(a.c.eps)) // self pairs masked, as the tail
-      tile_pass<R, U, false, true, true, PRIO>(L, src, w, lane, a.c.eps, vt, B * P,
-                                         n, s0, s1);
-    else if (masked)
-      tile_pass<R, U, false, R::MASKED_TAIL, false, PRIO>(L, src, w, lane,
-                                                          a.c.eps, vt,
-                                             B * P, n, s0, s1);
-    else
-      tile_pass<R, U, false, false, false, PRIO>(L, src, w, lane, a.c.eps,
-                                                 vt, B * P, n, s0, s1);
-  } else {
-#pragma unroll
-    for (int q = 0; q < U; ++q)
-#pragma unroll
-      for (int e = 0; e < R::ACC; ++e) L.rs[q][e] = 0.0f;
-    if (masked)
-      tile_pass<R, U, true, R::MASKED_TAIL, false, PRIO>(L, src, w, lane,
-                                                         a.c.eps, vt,
-                                            B * P, n, s0, s1);
-    else
-      tile_pass<R, U, true, false, false, PRIO>(L, src, w, lane, a.c.eps, vt,
-                                                B * P, n, s0, s1);
-    // after the rotations of steps [s0, s1) lane l holds the sums of source
-    // set (l + s1) mod 64 (set l again after a whole pass)
-    float *sp = slot + R::ACC * P + ((lane + s1) & 63) * U;
-#pragma unroll
-    for (int q = 0; q < U; ++q)
-#pragma unroll
-      for (int e = 0; e < R::ACC; ++e) sp[e * P + q] = L.rs[q][e];
-  }
-  float *fp = slot + lane * U;
-#pragma unroll
-  for (int k = 0; k < U; ++k)
-#pragma unroll
-    for (int e = 0; e < R::ACC; ++e) fp[e * P + k] = L.a[k][e];
-}
-
-// Per particle: row partials of its tile (B order) minus the negated
-// reaction partials of its column (A order), in kTileRuns runs; then the
-// rule's epilogue.
-template <class R, int U, int HALVES = 1>
-__global__ __launch_bounds__(256) void sym_tile_finalize(SymArgs a) {
-  constexpr int P = 64 * U;
-  constexpr int PW = 256 / kTileRuns; // particles per workgroup
-  __shared__ float red[R::ACC][256];
-  const int i = blockIdx.x * PW + threadIdx.x % PW;
-  const int run = threadIdx.x / PW;
-  const bool live = i < a.n;
-  float f[R::ACC];
-  if (live) {
-    const int g = i / P, o = i % P, T = a.ts;
-    // rows of pairs (g, g + k / HALVES), then the reactions of (c / HALVES,
-    // g), each pair's halves in order
-    run_sum<R, kTileRuns>(
-        f, HALVES * (T - g), HALVES * g, run,
-        [&](int k) {
-          const long long it = tri_slot(g, g + k / HALVES, T) * HALVES + k % HALVES;
-          return a.fpart + (size_t)it * (2 * R::ACC * P) + o;
-        },
-        [&](int c) {
-          const long long it = tri_slot(c / HALVES, g, T) * HALVES + c % HALVES;
-          return a.fpart + (size_t)it * (2 * R::ACC * P) + R::ACC * P + o;
-        },
-        P);
-  } else {
-#pragma unroll
-    for (int e = 0; e < R::ACC; ++e) f[e] = 0.0f;
-  }
-  if (combine_runs<R, kTileRuns>(f, red) && live) R::finish(a, i, f);
 }
 
 // ---- many independent systems (batched persistent launch) ----------------
@@ -1161,6 +1252,28 @@ __device__ __forceinline__ SymArgs system_view(const SymBatchArgs &b, int s,
   return a;
 }
 
+// The queue of a persistent grid: every thread of the workgroup gets the next
+// item, or one >= num_items when the queue is drained.
+__device__ __forceinline__ int next_item(const SymBatchArgs &b, int *s_item) {
+  if (threadIdx.x == 0) *s_item = atomicAdd(b.counters, 1);
+  __syncthreads();
+  const int item = *s_item;
+  __syncthreads(); // every lane has read s_item before it is rewritten
+  return item;
+}
+
+// The last workgroup to leave resets the counters for the next launch.
+__device__ __forceinline__ void leave_queue(const SymBatchArgs &b) {
+  if (threadIdx.x == 0) {
+    __threadfence(); // this workgroup's last queue access precedes the count
+    const int done = atomicAdd(b.counters + 1, 1);
+    if (done == (int)gridDim.x - 1) {
+      atomicExch(b.counters, 0);
+      atomicExch(b.counters + 1, 0);
+    }
+  }
+}
+
 template <int U>
 __global__ __launch_bounds__(256) void sym_batch_kernel(SymBatchArgs b) {
   using R = ForceRule;
@@ -1173,10 +1286,7 @@ __global__ __launch_bounds__(256) void sym_batch_kernel(SymBatchArgs b) {
   float *sacc = reinterpret_cast<float *>(sacc4);
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (;;) {
-    if (threadIdx.x == 0) s_item = atomicAdd(b.counters, 1);
-    __syncthreads();
-    const int item = s_item;
-    __syncthreads(); // every lane has read s_item before it is rewritten
+    const int item = next_item(b, &s_item);
     if (item >= b.num_items) break;
     const int4 it = b.items[item];
     const SymArgs a = system_view(b, it.x, ST);
@@ -1187,20 +1297,32 @@ __global__ __launch_bounds__(256) void sym_batch_kernel(SymBatchArgs b) {
     pair_step(T, vt, a, src, sacc, it.y, it.z, slot + R::ACC * ST);
     store_row(T, slot, w, lane);
   }
-  if (threadIdx.x == 0) {
-    __threadfence(); // this workgroup's last queue access precedes the count
-    const int done = atomicAdd(b.counters + 1, 1);
-    if (done == (int)gridDim.x - 1) {
-      atomicExch(b.counters, 0);
-      atomicExch(b.counters + 1, 0);
-    }
-  }
+  leave_queue(b);
 }
 
+// The same in the row form (U targets per lane, ST = 64 U).
 template <int U>
+__global__ __launch_bounds__(256, 4) void sym_row_batch_kernel(SymBatchArgs b) {
+  using R = ForceRule;
+  constexpr int ST = RowShape<R, U>::ST;
+  __shared__ float lds[RowShape<R, U>::LDS_FLOATS];
+  __shared__ int s_item;
+  for (;;) {
+    // its barriers also hold the item's LDS until every wave is done with it
+    const int item = next_item(b, &s_item);
+    if (item >= b.num_items) break;
+    const int4 it = b.items[item];
+    const SymArgs a = system_view(b, it.x, ST);
+    float *slot = b.part + (size_t)it.w * (2 * R::ACC * ST);
+    row_item<R, U>(a, lds, it.y, it.z, it.z + 1, slot,
+                   [&](int) { return slot + R::ACC * ST; });
+  }
+  leave_queue(b);
+}
+
+template <int ST>
 __global__ __launch_bounds__(256) void sym_batch_finalize(SymBatchArgs b) {
   using R = ForceRule;
-  constexpr int ST = kWaves * 64 * U;
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= b.total) return;
   // system of particle i: the last s with sys_off[s] <= i (empty systems
@@ -1231,46 +1353,48 @@ __global__ __launch_bounds__(256) void sym_batch_finalize(SymBatchArgs b) {
 
 using KernelFn = void (*)(SymArgs);
 
+// Kernels of one launch shape and its super-tile.  runs: finalize runs per
+// particle.
 struct SymShape {
-  int unroll;
+  int st, runs;
   KernelFn pairs, finalize;
 };
 
-template <class R>
-const SymShape *find_shape(int unroll, bool tiles) {
-  static const SymShape shapes[] = {
-      {2, sym_kernel<R, 2>, sym_finalize<R, 2>},
-      {4, sym_kernel<R, 4>, sym_finalize<R, 4>},
-      {8, sym_kernel<R, 8>, sym_finalize<R, 8>},
-  };
-  static const SymShape tile_shapes[] = {
-      {2, sym_tile_kernel<R, 2>, sym_tile_finalize<R, 2>},
-      {4, sym_tile_kernel<R, 4>, sym_tile_finalize<R, 4>},
-  };
-  if (tiles) {
-    for (const SymShape &s : tile_shapes)
-      if (s.unroll == unroll) return &s;
-    return nullptr;
-  }
-  for (const SymShape &s : shapes)
-    if (s.unroll == unroll) return &s;
-  return nullptr;
+template <class R, int U, int RUNS>
+constexpr SymShape row_shape() {
+  return {64 * U, RUNS, sym_row_kernel<R, U>, sym_finalize<R, 64 * U, RUNS>};
 }
 
-// Kahan shapes: 2 or 4 per lane (the compensations double the sums).
-const SymShape *find_kahan_shape(int unroll, bool tiles) {
-  using R = KahanForceRule;
-  static const SymShape shapes[] = {
-      {2, sym_kernel<R, 2>, sym_finalize<R, 2>},
-      {4, sym_kernel<R, 4>, sym_finalize<R, 4>},
-  };
-  static const SymShape tile_shapes[] = {
-      {2, sym_tile_kernel<R, 2>, sym_tile_finalize<R, 2>},
-      {4, sym_tile_kernel<R, 4>, sym_tile_finalize<R, 4>},
-  };
-  for (int k = 0; k < 2; ++k) {
-    const SymShape &s = tiles ? tile_shapes[k] : shapes[k];
-    if (s.unroll == unroll) return &s;
+template <class R, int U>
+constexpr SymShape wave_shape() {
+  return {256 * U, 1, sym_kernel<R, U>, sym_finalize<R, 256 * U, 1>};
+}
+
+// Targets per lane of a tile-pair shape: `unroll` particles per lane and
+// tile (tiles of 64 * unroll), `items` work items per tile pair.  Tiles of 2
+// per lane are taken two at a time (4 targets per lane), one at a time with
+// two items per tile pair.
+int tile_targets(int unroll, int items) {
+  return unroll == 2 && items == 1 ? 4 : unroll;
+}
+
+// Super-tiles of 512 (2 per lane) run in the row form, larger ones in the
+// four-wave form; tile pairs in the row form with one super-tile per tile or
+// pair of tiles.
+template <class R>
+const SymShape *find_shape(int unroll, bool tiles, int items) {
+  static const SymShape row2 = row_shape<R, 2, kTileRuns>(),
+                        row4 = row_shape<R, 4, kTileRuns>(),
+                        row8 = row_shape<R, 8, 1>(), wave4 = wave_shape<R, 4>();
+  if (tiles) {
+    if (unroll != 2 && unroll != 4) return nullptr;
+    return tile_targets(unroll, items) == 2 ? &row2 : &row4;
+  }
+  if (unroll == 2) return &row8;
+  if (unroll == 4) return &wave4;
+  if constexpr (R::WAVE8) {
+    static const SymShape wave8 = wave_shape<R, 8>();
+    if (unroll == 8) return &wave8;
   }
   return nullptr;
 }
@@ -1284,31 +1408,25 @@ bool sym_banded(int unroll, bool tiles, int chunk, int acc, size_t n) {
 }
 
 struct BandShape {
-  int unroll;
+  int unroll, st;
   KernelFn pairs, fold, finish;
 };
 
-template <class R, int U>
-BandShape band_shape() {
-  return {U, sym_band_kernel<R, U>, sym_band_fold<R, U>, sym_band_finish<R, U>};
-}
-
-// Band kernels of rule R: 2, 4 or 8 particles per lane (Kahan: 2 or 4).
+// Band kernels of rule R: 2 (row form), 4 or 8 particles per lane (Kahan: 2
+// or 4).
 template <class R>
 const BandShape *find_band_shape(int unroll) {
-  static const BandShape shapes[] = {band_shape<R, 2>(), band_shape<R, 4>(),
-                                     band_shape<R, 8>()};
-  for (const BandShape &s : shapes)
-    if (s.unroll == unroll) return &s;
-  return nullptr;
-}
-
-template <>
-const BandShape *find_band_shape<KahanForceRule>(int unroll) {
-  static const BandShape shapes[] = {band_shape<KahanForceRule, 2>(),
-                                     band_shape<KahanForceRule, 4>()};
-  for (const BandShape &s : shapes)
-    if (s.unroll == unroll) return &s;
+  static const BandShape b2 = {2, 512, sym_row_band_kernel<R, 8>,
+                               sym_band_fold<R, 512>, sym_band_finish<R>},
+                         b4 = {4, 1024, sym_band_kernel<R, 4>,
+                               sym_band_fold<R, 1024>, sym_band_finish<R>};
+  if (unroll == 2) return &b2;
+  if (unroll == 4) return &b4;
+  if constexpr (R::WAVE8) {
+    static const BandShape b8 = {8, 2048, sym_band_kernel<R, 8>,
+                                 sym_band_fold<R, 2048>, sym_band_finish<R>};
+    if (unroll == 8) return &b8;
+  }
   return nullptr;
 }
 
@@ -1339,9 +1457,8 @@ BandPlan band_plan(size_t n, int unroll, int chunk) {
 
 int launch_sym_banded(const BandShape *band, SymArgs &a, int chunk, int n,
                       float *scratch, int acc, hipStream_t stream) {
-  const int unroll = band->unroll;
-  const int st = kWaves * 64 * unroll;
-  const BandPlan bp = band_plan((size_t)n, unroll, chunk);
+  const int st = band->st;
+  const BandPlan bp = band_plan((size_t)n, band->unroll, chunk);
   if (bp.w < 1)
     return set_error(NB_ERR_UNSUPPORTED, "no band plan for this size");
   a.fpart = scratch;
@@ -1397,27 +1514,18 @@ int launch_sym(const SymShape *sh, SymArgs &a, int unroll, int chunk, int n,
     return set_error(NB_ERR_UNSUPPORTED, "no symmetric kernel for this shape");
   if (!scratch)
     return set_error(NB_ERR_INVALID_ARG, "symmetric launch needs scratch");
-  long long blocks;
   if (tiles) {
     if (chunk > 2)
       return set_error(NB_ERR_UNSUPPORTED,
                        "tile-pair shapes take one or two items per tile pair");
-    const int P = 64 * unroll;
-    const int T = (n + P - 1) / P;
-    a.fpart = scratch;
-    a.spart = nullptr;
-    a.ts = T;
-    a.chunk = chunk; // items per tile pair
-    blocks = ((long long)chunk * T * (T + 1) / 2 + kWaves - 1) / kWaves;
-  } else {
-    const int st = kWaves * 64 * unroll;
-    const int ts = (n + st - 1) / st;
-    blocks = items_upto(ts, chunk);
-    a.fpart = scratch;
-    a.spart = scratch + (size_t)blocks * acc * st;
-    a.ts = ts;
-    a.chunk = chunk;
+    chunk = 1; // one super-tile pair per work item
   }
+  const int ts = (n + sh->st - 1) / sh->st;
+  const long long blocks = items_upto(ts, chunk);
+  a.fpart = scratch;
+  a.spart = scratch + (size_t)blocks * acc * sh->st;
+  a.ts = ts;
+  a.chunk = chunk;
   a.n = n;
   void *args[] = {&a};
   int r = hip_check(hipLaunchKernel(reinterpret_cast<const void *>(sh->pairs),
@@ -1425,7 +1533,7 @@ int launch_sym(const SymShape *sh, SymArgs &a, int unroll, int chunk, int n,
                                     stream),
                     "symmetric pair launch");
   if (r) return r;
-  const int per_block = tiles ? 256 / kTileRuns : 256;
+  const int per_block = 256 / sh->runs;
   return hip_check(
       hipLaunchKernel(reinterpret_cast<const void *>(sh->finalize),
                       dim3((n + per_block - 1) / per_block), dim3(256), args,
@@ -1439,10 +1547,15 @@ size_t sym_scratch_bytes(int unroll, int chunk, size_t n, int acc,
                          bool tiles, bool bandable) {
   if (tiles) {
     if (n == 0 || n > sym_max_particles(unroll, tiles, chunk, acc)) return 0;
+    // the limits of the callers' buffers are stated in tile pairs: a row and a
+    // reaction partial per pair and item; the row form needs no more from the
+    // second tile on
     const long long P = 64LL * unroll;
     const long long T = ((long long)n + P - 1) / P;
-    return sizeof(float) * (size_t)(T * (T + 1) / 2) * 2 * acc * (size_t)P *
-           (size_t)std::max(chunk, 1);
+    const long long st = 64LL * tile_targets(unroll, chunk);
+    const long long ts = ((long long)n + st - 1) / st;
+    return sizeof(float) * acc *
+           (size_t)std::max(T * (T + 1) * P * std::max(chunk, 1), ts * ts * st);
   }
   if (bandable && sym_banded(unroll, tiles, chunk, acc, n)) {
     const BandPlan bp = band_plan(n, unroll, chunk);
@@ -1491,10 +1604,13 @@ int sym_batch_layout(int unroll, const int *sys_off, int num_systems,
 
 namespace {
 template <int U> const void *batch_pairs_fn() {
-  return reinterpret_cast<const void *>(sym_batch_kernel<U>);
+  if constexpr (U == 2)
+    return reinterpret_cast<const void *>(sym_row_batch_kernel<8>);
+  else
+    return reinterpret_cast<const void *>(sym_batch_kernel<U>);
 }
 template <int U> const void *batch_finalize_fn() {
-  return reinterpret_cast<const void *>(sym_batch_finalize<U>);
+  return reinterpret_cast<const void *>(sym_batch_finalize<kWaves * 64 * U>);
 }
 } // namespace
 
@@ -1565,64 +1681,14 @@ int launch_forward_sym(const StepConsts &c, int unroll, int chunk, bool tiles,
   if (tiles && chunk != 1 && (kahan || unroll != 2))
     return set_error(NB_ERR_UNSUPPORTED,
                      "two items per tile pair: plain sums, 2 per lane only");
-  // Kahan tile pairs with the priority steps up to n = 16384 (same results
-  // bit for bit): 12288 76.2-76.5 vs 79.8-80.0 us, 16384 118.8-118.9 vs
-  // 119.4-119.5 us; from 20480 on 2-5 % slower (more work per wave).
-  if (kahan && tiles && unroll == 2 && (size_t)n <= kKahanTilePrioMaxParticles) {
-    static const SymShape kprio = {2, sym_tile_kernel<KahanForceRule, 2, true>,
-                                   sym_tile_finalize<KahanForceRule, 2>};
-    return launch_sym(&kprio, a, unroll, chunk, n, scratch, KahanForceRule::ACC,
-                      tiles, stream, nullptr);
-  }
   if (kahan)
     return launch_sym(
-        find_kahan_shape(unroll, tiles), a, unroll, chunk, n, scratch,
-        KahanForceRule::ACC, tiles, stream,
+        find_shape<KahanForceRule>(unroll, tiles, chunk), a, unroll, chunk, n,
+        scratch, KahanForceRule::ACC, tiles, stream,
         tiles ? nullptr : find_band_shape<KahanForceRule>(unroll));
-  // Tile pairs of 2 per lane up to n = 32768 with the quarter-pass priority
-  // steps (PRIO in tile_pass; same results bit for bit): n = 4096 20.6 vs
-  // 23.8 us, 8192 30.6 vs 31.4 us, 12800 47.4 vs 49.2 us; with the priority
-  // set outside the step loop also 14336 56.5-57.5 vs 59.6-60.3 us, 20480
-  // 94.5-96.8 vs 97.2-98.5 us, 25600 and 32768 about 1 % faster, 16384 the
-  // same, 40960 0.3 % slower.
-  // Two items per tile pair (forward config 37, the default at 4096 <= n <
-  // 6656) against one item with priority steps: n = 4096 15.5 vs 20.0 us,
-  // 6144 20.9 vs 22.2 us; from 7168 on the doubled partials cost more than
-  // the balance gains (7168 24.6 vs 23.1 us, 8192 28.6 vs 27.2 us, 12800
-  // 47.2 vs 42.5 us).  The half items take the priority steps as well (per
-  // quarter of their 32 steps): 4096 15.1-15.4 vs 15.4-15.5 us, 5120
-  // 16.5-16.8 vs 17.0-17.1 us, 6144 19.8-19.9 vs 20.9-21.0 us.
-  if (tiles && unroll == 2 && chunk == 2) {
-    static const SymShape halves = {2, sym_tile_kernel<ForceRule, 2, true, 2>,
-                                    sym_tile_finalize<ForceRule, 2, 2>};
-    return launch_sym(&halves, a, unroll, chunk, n, scratch, ForceRule::ACC,
-                      tiles, stream, nullptr);
-  }
-  if (tiles && unroll == 2 && (size_t)n <= kTilePrioMaxParticles) {
-    static const SymShape prio = {2, sym_tile_kernel<ForceRule, 2, true>,
-                                  sym_tile_finalize<ForceRule, 2>};
-    return launch_sym(&prio, a, unroll, chunk, n, scratch, ForceRule::ACC,
-                      tiles, stream, nullptr);
-  }
-  return launch_sym(find_shape<ForceRule>(unroll, tiles), a, unroll, chunk, n,
-                    scratch, ForceRule::ACC, tiles, stream,
+  return launch_sym(find_shape<ForceRule>(unroll, tiles, chunk), a, unroll,
+                    chunk, n, scratch, ForceRule::ACC, tiles, stream,
                     tiles ? nullptr : find_band_shape<ForceRule>(unroll));
-}
-
-// The adjoint's tile pairs of 2 per lane take the quarter-pass priority
-// steps too (same results bit for bit): adjoint / fused n = 8192 39.9-40.3 vs
-// 43.3-44.1 us / 47.8-48.2 vs 51.1-51.4 us, 12800 59.8-60.3 vs 63.6-64.1 /
-// 75.8-76.2 vs 80.3-80.4, 16384 95.7-96.1 vs 99.3-99.9 / 120.4-120.6 vs
-// 125.3-125.5, 20000 135.4-135.9 vs 137.3-139.2 / 173.3-173.5 vs 177.8-177.9;
-// 2048 and 4096 the same.
-template <bool F>
-const SymShape *adjoint_shape(int unroll, bool tiles, int n) {
-  if (tiles && unroll == 2 && (size_t)n <= kTilePrioMaxParticles) {
-    static const SymShape prio = {2, sym_tile_kernel<AdjointRule<F>, 2, true>,
-                                  sym_tile_finalize<AdjointRule<F>, 2>};
-    return &prio;
-  }
-  return find_shape<AdjointRule<F>>(unroll, tiles);
 }
 
 int launch_adjoint_sym(const StepConsts &c, bool fused, int unroll, int chunk,
@@ -1651,11 +1717,11 @@ int launch_adjoint_sym(const StepConsts &c, bool fused, int unroll, int chunk,
     a.ny = nxt[1];
     a.nz = nxt[2];
     return launch_sym(
-        adjoint_shape<true>(unroll, tiles, n), a, unroll, chunk, n,
+        find_shape<AdjointRule<true>>(unroll, tiles, chunk), a, unroll, chunk, n,
         scratch, AdjointRule<true>::ACC, tiles, stream,
         tiles ? nullptr : find_band_shape<AdjointRule<true>>(unroll));
   }
-  return launch_sym(adjoint_shape<false>(unroll, tiles, n), a, unroll,
+  return launch_sym(find_shape<AdjointRule<false>>(unroll, tiles, chunk), a, unroll,
                     chunk, n, scratch, AdjointRule<false>::ACC, tiles, stream,
                     tiles ? nullptr : find_band_shape<AdjointRule<false>>(unroll));
 }
