@@ -231,7 +231,8 @@ int configure_sym(nb_batch *b, int cfg) {
   b->num_items = (int)items.size();
   int per_cu = 0;
   if ((st = hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                          &per_cu, sym_batch_kernel_fn(sh.unroll), 256, 0),
+                          &per_cu, sym_batch_kernel_fn(sh.unroll),
+                          sym_batch_threads(sh.unroll), 0),
                       "occupancy query")))
     return st;
   b->grid = std::max(1, std::min(b->num_items, std::max(1, per_cu) * b->num_cu));

@@ -137,8 +137,10 @@ struct SymBatchLaunch {
   int *counters; // two self-resetting queue counters (zero before first use)
   int grid;      // persistent workgroups
 };
-// Pair kernel of the batched symmetric step (for occupancy queries).
+// Pair kernel of the batched symmetric step and its workgroup size (for
+// occupancy queries).
 const void *sym_batch_kernel_fn(int unroll);
+int sym_batch_threads(int unroll);
 int launch_sym_batch(int unroll, const SymBatchLaunch &L, hipStream_t stream);
 
 int launch_forward_sym(const StepConsts &c, int unroll, int chunk, bool tiles,

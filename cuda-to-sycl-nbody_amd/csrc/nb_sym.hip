@@ -25,37 +25,20 @@
 // particle, its row partials in chunk order, then subtracts the reaction
 // partials of its column in GA order, and applies the rule's epilogue.  The
 // order is fixed: results are deterministic.
-// Two forms of the pair kernel:
-//   * row form (sym_row_kernel; ST = 128, 256, 512): a wave holds all
-//     targets of GA and meets GB in sets of 64 sources (see row_item).  The
-//     shapes with 2 particles per lane of the workgroup (ST = 512) and the
-//     tile pairs;
-//   * four-wave form (sym_kernel; U = 4 or 8 per lane, P = 64 U per wave, ST =
-//     4 P): wave w holds targets 4 GA + w (tile of P) in VGPRs; the source
-//     super-tile sits in LDS; for GB > GA, in pass b wave w meets source tile
-//     j = (w + b) & 3; in each of 64 steps lane l takes the U sources of set
-//     (l + s) & 63 from LDS and evaluates the U x U pair terms, adding the
-//     (negated) reaction to U per-source sums that rotate one lane down the
-//     wave (wave_rol1 or lds_rol1) after each step, so that after 64 steps
-//     lane l again holds set l's sums.  Between passes the reaction sums of
-//     the four tiles live in LDS (each tile is owned by one wave per pass).
-//     For GB == GA each wave meets its own tile without reactions (self terms
-//     are +0) and then, with 4 per lane, the tiles above it with reactions
-//     (each of the six tile pairs once), subtracting at the end the reactions
-//     its tile received; with 8 per lane it meets the other three tiles
-//     without reactions as well.  A quarter of the row form's reaction
-//     partials per pair: the choice where those dominate (n >= 2^18).
+// Inside an item a wave holds all targets of one row of GA (64 U, U = 8, 4 or
+// 2 per lane) and meets GB in sets of 64 sources; a set's reaction sums rotate
+// one lane down the wave after each step (meet_sources).
 // The super-tile pairs of many independent systems also run on one
-// persistent queue (sym_batch_kernel, sym_row_batch_kernel).
+// persistent queue (sym_batch_kernel).
 // Padding (index >= n): ForceRule puts padding particles at 1e30 in every
 // coordinate, so any pair with a real particle has |r|^2 = +inf,
 // rsqrt(inf) = 0 and r * 0 = 0 (exact zeros, no mask; a pair of two padding
 // particles only touches padding sums).  AdjointRule masks K and t3 of pairs
-// with a padding particle in the items that contain the last, partial
-// (super-)tile (a product r . h of a far padding particle could overflow).
+// with a padding particle in the last, partial set of sources (a product
+// r . h of a far padding particle could overflow).
 // Self pairs: with dist_eps^3 a normal float the self term is exactly +0
-// (r = 0, finite K); otherwise (eps = 0 or tiny) the pass of each wave over
-// its own tile, the only one holding self pairs, masks them as the
+// (r = 0, finite K); otherwise (eps = 0 or tiny) the passes over the
+// super-tile's own sets, the only ones holding self pairs, mask them as the
 // reference's `continue` skips them.
 //
 // Per pair term (two interactions): forward 14 VALU + v_rsq_f32 + 3/U
@@ -76,32 +59,14 @@
 namespace nb {
 namespace {
 
-constexpr int kWaves = 4;        // waves per workgroup = tiles per super-tile
 constexpr float kFar = 1.0e30f;  // coordinate of ForceRule padding particles
-constexpr int kDppWaveRol1 = 0x134;
 
-// Lane l receives lane (l + 1) mod 64's value.  Two forms of the same move:
-//   wave_rol1  a DPP wave_rol:1 move on the VALU.  Every lane is written
-//              (full row and bank masks), so the "old" operand is the source
-//              itself: with a constant there the compiler materialises it
-//              with an extra v_mov per call;
-//   lds_rol1   ds_bpermute_b32 through the LDS crossbar (no LDS memory): it
-//              takes no VALU issue slot.  Inside the pair loop's mix a DPP
-//              move costs about as much VALU time as a v_rsq_f32 (10-14 SIMD
-//              cycles, measured with probe/issue_rates.hip), while the
-//              permute's latency is hidden (each sum is rotated as soon as
-//              it is complete and read again only in the next step).  The
-//              row form and the forward rules rotate with lds_rol1; the
-//              adjoint rules' four-wave form, whose loop reads twice the LDS
-//              per step already, keeps DPP for the adjoint sums (lds_rol1
-//              for all of them measured 1.5 % slower for the adjoint, 4 % for
-//              the fused step).
-__device__ __forceinline__ float wave_rol1(float v) {
-  const int b = __builtin_bit_cast(int, v);
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_update_dpp(b, b, kDppWaveRol1, 0xf, 0xf, false));
-}
-
+// Lane l receives lane (l + 1) mod 64's value: ds_bpermute_b32 through the LDS
+// crossbar (no LDS memory).  It takes no VALU issue slot; a DPP move
+// (wave_rol:1) costs 10-14 SIMD cycles of VALU time inside the pair loop's mix
+// (measured with probe/issue_rates.hip), while the permute's latency is hidden
+// (each sum is rotated as soon as it is complete and read again only in the
+// next step).
 __device__ __forceinline__ float lds_rol1(float v) {
   const int lane =
       (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
@@ -170,25 +135,13 @@ struct PlainPartials {
 #pragma unroll
     for (int e = 0; e < ACC; ++e) f[e] = f[e] - v[e];
   }
-  static __device__ __forceinline__ void sub_reaction(float (&f)[ACC],
-                                                      const float *p,
-                                                      int stride) {
-    float v[ACC];
-    fetch(v, p, stride);
-    sub_v(f, v);
-  }
 };
 
 struct ForceRule : PlainPartials<3> {
   static constexpr int SRC = 3; // x, y, z
   static constexpr int ACC = 3; // F
   static constexpr bool MASKED_TAIL = false;
-  // every sum rotates with lds_rol1 (see wave_rol1)
-  static constexpr bool rotate_lds(int) { return true; }
-  // the four-wave super-tile passes run the pair term as a block of assembly
-  // per source (nb_pair_block.hpp); the row form does for every rule
-  static constexpr bool BLOCK = true;
-  static constexpr bool WAVE8 = true; // four-wave kernels with 8 per lane
+  static constexpr bool ROWS4 = true; // has shapes with 8 per lane
 
   template <int U>
   static __device__ __forceinline__ void block(const float (&s)[SRC],
@@ -206,17 +159,15 @@ struct ForceRule : PlainPartials<3> {
     v[2] = ok ? a.pz[j] : kFar;
   }
 
-  // Source s on target t: a += r K.  With SYM, rs accumulates +r K too: rs
-  // holds the negated reaction sum of the source (the finalize subtracts it),
-  // which keeps every accumulation a two-operand v_fmac_f32.  With MASK the
-  // term of a pair that is not `valid` is zero (the self pair when eps^3 is
-  // not a normal float, as the reference's `continue` skips it).
-  template <bool SYM, bool MASK>
-  static __device__ __forceinline__ void pair(const float (&s)[SRC],
-                                              const float (&t)[SRC],
-                                              float (&a)[ACC],
-                                              float (&rs)[ACC], float eps,
-                                              bool valid) {
+  // Source s on target t: a += r K and rs += r K: rs holds the negated
+  // reaction sum of the source (the finalize subtracts it), which keeps every
+  // accumulation a two-operand v_fmac_f32.  The term of a pair that is not
+  // `valid` is zero (the self pair when eps^3 is not a normal float, as the
+  // reference's `continue` skips it; pairs with padding where a rule needs
+  // it).  block() is the same without the mask, for U targets.
+  static __device__ __forceinline__ void
+  pair_masked(const float (&s)[SRC], const float (&t)[SRC], float (&a)[ACC],
+              float (&rs)[ACC], float eps, bool valid) {
     const float rx = s[0] - t[0];
     const float ry = s[1] - t[1];
     const float rz = s[2] - t[2];
@@ -224,15 +175,13 @@ struct ForceRule : PlainPartials<3> {
     d = __builtin_fmaf(ry, ry, d);
     d = __builtin_fmaf(rz, rz, d);
     float K = __builtin_amdgcn_rsqf((d * d) * d);
-    if constexpr (MASK) K = valid ? K : 0.0f;
+    K = valid ? K : 0.0f;
     a[0] = __builtin_fmaf(rx, K, a[0]);
     a[1] = __builtin_fmaf(ry, K, a[1]);
     a[2] = __builtin_fmaf(rz, K, a[2]);
-    if constexpr (SYM) {
-      rs[0] = __builtin_fmaf(rx, K, rs[0]);
-      rs[1] = __builtin_fmaf(ry, K, rs[1]);
-      rs[2] = __builtin_fmaf(rz, K, rs[2]);
-    }
+    rs[0] = __builtin_fmaf(rx, K, rs[0]);
+    rs[1] = __builtin_fmaf(ry, K, rs[1]);
+    rs[2] = __builtin_fmaf(rz, K, rs[2]);
   }
 
   static __device__ __forceinline__ void finish(const SymArgs &a, int i,
@@ -248,8 +197,7 @@ struct ForceRule : PlainPartials<3> {
 // sum is s - c).  A partial is (s_x, s_y, s_z, c_x, c_y, c_z); the finalize
 // Kahan-adds the partials' values s - c.
 struct KahanForceRule {
-  static constexpr bool BLOCK = false;
-  static constexpr bool WAVE8 = false;
+  static constexpr bool ROWS4 = false;
   static constexpr int SRC = 3;
   static constexpr int ACC = 6;
 
@@ -262,20 +210,15 @@ struct KahanForceRule {
   }
 
   static constexpr bool MASKED_TAIL = false;
-  // every sum rotates with lds_rol1 (see wave_rol1)
-  static constexpr bool rotate_lds(int) { return true; }
 
   static __device__ __forceinline__ void load(const SymArgs &a, int j,
                                               float (&v)[SRC]) {
     ForceRule::load(a, j, v);
   }
 
-  template <bool SYM, bool MASK>
-  static __device__ __forceinline__ void pair(const float (&s)[SRC],
-                                              const float (&t)[SRC],
-                                              float (&a)[ACC],
-                                              float (&rs)[ACC], float eps,
-                                              bool valid) {
+  static __device__ __forceinline__ void
+  pair_masked(const float (&s)[SRC], const float (&t)[SRC], float (&a)[ACC],
+              float (&rs)[ACC], float eps, bool valid) {
     const float rx = s[0] - t[0];
     const float ry = s[1] - t[1];
     const float rz = s[2] - t[2];
@@ -283,15 +226,13 @@ struct KahanForceRule {
     d = __builtin_fmaf(ry, ry, d);
     d = __builtin_fmaf(rz, rz, d);
     float K = __builtin_amdgcn_rsqf((d * d) * d);
-    if constexpr (MASK) K = valid ? K : 0.0f; // as ForceRule
+    K = valid ? K : 0.0f; // as ForceRule
     kahan_add(rx, K, a[0], a[3]);
     kahan_add(ry, K, a[1], a[4]);
     kahan_add(rz, K, a[2], a[5]);
-    if constexpr (SYM) {
-      kahan_add(rx, K, rs[0], rs[3]);
-      kahan_add(ry, K, rs[1], rs[4]);
-      kahan_add(rz, K, rs[2], rs[5]);
-    }
+    kahan_add(rx, K, rs[0], rs[3]);
+    kahan_add(ry, K, rs[1], rs[4]);
+    kahan_add(rz, K, rs[2], rs[5]);
   }
 
   // f: running (sum, compensation) of each coordinate over the partials
@@ -317,13 +258,6 @@ struct KahanForceRule {
 #pragma unroll
     for (int e = 0; e < 3; ++e) kahan_value(f, e, v[3 + e] - v[e]);
   }
-  static __device__ __forceinline__ void sub_reaction(float (&f)[ACC],
-                                                      const float *p,
-                                                      int stride) {
-    float v[ACC];
-    fetch(v, p, stride);
-    sub_v(f, v);
-  }
 
   static __device__ __forceinline__ void finish(const SymArgs &a, int i,
                                                 const float (&f)[ACC]) {
@@ -334,8 +268,7 @@ struct KahanForceRule {
 
 template <bool FUSED>
 struct AdjointRule : PlainPartials<FUSED ? 6 : 3> {
-  static constexpr bool BLOCK = false;
-  static constexpr bool WAVE8 = true;
+  static constexpr bool ROWS4 = true;
   static constexpr int SRC = 6; // x, y, z, g_x, g_y, g_z
   static constexpr int ACC = FUSED ? 6 : 3; // sum M (g_j - g_k) [, F]
   static constexpr bool MASKED_TAIL = true;
@@ -348,10 +281,6 @@ struct AdjointRule : PlainPartials<FUSED ? 6 : 3> {
     if constexpr (FUSED) fused_block<U>(s, t, a, rs, eps);
     else adjoint_block<U>(s, t, a, rs, eps);
   }
-
-  // four-wave form: the adjoint sums rotate by DPP, the fused step's force
-  // sums (3..5) with lds_rol1
-  static constexpr bool rotate_lds(int c) { return FUSED && c >= 3; }
 
   // g = lv' + dt lx' (the cotangent the pair sum is taken of)
   static __device__ __forceinline__ void load(const SymArgs &a, int j,
@@ -369,12 +298,9 @@ struct AdjointRule : PlainPartials<FUSED ? 6 : 3> {
     }
   }
 
-  template <bool SYM, bool MASK>
-  static __device__ __forceinline__ void pair(const float (&s)[SRC],
-                                              const float (&t)[SRC],
-                                              float (&a)[ACC],
-                                              float (&rs)[ACC], float eps,
-                                              bool valid) {
+  static __device__ __forceinline__ void
+  pair_masked(const float (&s)[SRC], const float (&t)[SRC], float (&a)[ACC],
+              float (&rs)[ACC], float eps, bool valid) {
     const float rx = s[0] - t[0];
     const float ry = s[1] - t[1];
     const float rz = s[2] - t[2];
@@ -400,30 +326,24 @@ struct AdjointRule : PlainPartials<FUSED ? 6 : 3> {
     rh = __builtin_fmaf(ry, hy, rh);
     rh = __builtin_fmaf(rz, hz, rh);
     float t3 = (rh * q) * -3.0f;
-    if constexpr (MASK) {
-      K = valid ? K : 0.0f;
-      t3 = valid ? t3 : 0.0f;
-    }
+    K = valid ? K : 0.0f;
+    t3 = valid ? t3 : 0.0f;
     const float ux = __builtin_fmaf(t3, rx, hx);
     const float uy = __builtin_fmaf(t3, ry, hy);
     const float uz = __builtin_fmaf(t3, rz, hz);
     a[0] = __builtin_fmaf(K, ux, a[0]);
     a[1] = __builtin_fmaf(K, uy, a[1]);
     a[2] = __builtin_fmaf(K, uz, a[2]);
-    if constexpr (SYM) { // negated reaction sums, as in ForceRule
-      rs[0] = __builtin_fmaf(K, ux, rs[0]);
-      rs[1] = __builtin_fmaf(K, uy, rs[1]);
-      rs[2] = __builtin_fmaf(K, uz, rs[2]);
-    }
+    rs[0] = __builtin_fmaf(K, ux, rs[0]); // negated, as in ForceRule
+    rs[1] = __builtin_fmaf(K, uy, rs[1]);
+    rs[2] = __builtin_fmaf(K, uz, rs[2]);
     if constexpr (FUSED) {
       a[3] = __builtin_fmaf(rx, K, a[3]);
       a[4] = __builtin_fmaf(ry, K, a[4]);
       a[5] = __builtin_fmaf(rz, K, a[5]);
-      if constexpr (SYM) {
-        rs[3] = __builtin_fmaf(rx, K, rs[3]);
-        rs[4] = __builtin_fmaf(ry, K, rs[4]);
-        rs[5] = __builtin_fmaf(rz, K, rs[5]);
-      }
+      rs[3] = __builtin_fmaf(rx, K, rs[3]);
+      rs[4] = __builtin_fmaf(ry, K, rs[4]);
+      rs[5] = __builtin_fmaf(rz, K, rs[5]);
     }
   }
 
@@ -442,256 +362,6 @@ struct AdjointRule : PlainPartials<FUSED ? 6 : 3> {
                     a.vz, a.nx, a.ny, a.nz);
   }
 };
-
-// LDS position of super-tile particle o (particle order o = j P + m U + q:
-// tile j, source set m, member q).  Within a tile, float4 slot qq * 64 + m
-// holds members 4 qq .. 4 qq + 3 of set m, so the 64 lanes of a step (sets
-// (l + s) mod 64, one quad each) read one contiguous 1 KiB block: no bank
-// conflicts.
-template <int U>
-__device__ __forceinline__ int lds_slot(int o) {
-  constexpr int P = 64 * U;
-  const int j = o / P, r = o % P;
-  const int m = r / U, q = r % U;
-  return j * P + (q >> 2) * 256 + m * 4 + (q & 3);
-}
-
-template <class R, int U>
-struct Lane {
-  float t[U][R::SRC];  // target inputs
-  float a[U][R::ACC];  // target sums
-  float rs[U][R::ACC]; // reaction sums of the current source set
-};
-
-// 64 steps of one wave against source tile j of the LDS super-tile (src:
-// R::SRC arrays of ST floats in lds_slot order; src0 = global index of the
-// tile's first particle).  With SYM the reaction sums rotate through the
-// wave.  With MASK, pairs with a padding particle contribute nothing (vt:
-// target validity; sources are valid below index n).  With SELF (a wave's
-// pass over its own tile, with MASK) the self pairs contribute nothing
-// either: needed when eps^3 is not a normal float.
-template <class R, int U, bool SYM, bool MASK, bool SELF = false>
-__device__ __forceinline__ void tile_pass(Lane<R, U> &L, const float *src,
-                                          int j, int lane, float eps,
-                                          const bool (&vt)[U], int src0,
-                                          int n) {
-  static_assert(!SELF || (MASK && !SYM), "self pairs: masked own-tile pass");
-  constexpr int P = 64 * U;
-  constexpr int ST = kWaves * P;
-  constexpr int Q = U / 4;
-  static_assert(U % 4 == 0, "particles per lane: a multiple of 4");
-  auto step = [&](int s) {
-    const int m = (lane + s) & 63;
-    float sv[U][R::SRC];
-#pragma unroll
-    for (int c = 0; c < R::SRC; ++c) {
-      const float4 *p4 = reinterpret_cast<const float4 *>(src + c * ST + j * P);
-#pragma unroll
-      for (int qq = 0; qq < Q; ++qq) {
-        const float4 v = p4[qq * 64 + m];
-        sv[4 * qq + 0][c] = v.x;
-        sv[4 * qq + 1][c] = v.y;
-        sv[4 * qq + 2][c] = v.z;
-        sv[4 * qq + 3][c] = v.w;
-      }
-    }
-    if constexpr (R::BLOCK && SYM && !MASK) {
-#pragma unroll
-      for (int q = 0; q < U; ++q) {
-        R::template block<U>(sv[q], L.t, L.a, L.rs[q], eps);
-#pragma unroll
-        for (int c = 0; c < R::ACC; ++c) L.rs[q][c] = lds_rol1(L.rs[q][c]);
-      }
-      return;
-    }
-#pragma unroll
-    for (int q = 0; q < U; ++q) {
-      const bool vs = !MASK || (src0 + m * U + q < n);
-#pragma unroll
-      for (int k = 0; k < U; ++k) {
-        // SELF (own tile): at step 0 member q of the lane's own set is its
-        // target q, the pair the reference skips
-        const bool self = SELF && s == 0 && q == k;
-        R::template pair<SYM, MASK>(sv[q], L.t[k], L.a[k], L.rs[q], eps,
-                                    vs && vt[k] && !self);
-      }
-    }
-    if constexpr (SYM) {
-#pragma unroll
-      for (int q = 0; q < U; ++q)
-#pragma unroll
-        for (int c = 0; c < R::ACC; ++c)
-          L.rs[q][c] =
-              R::rotate_lds(c) ? lds_rol1(L.rs[q][c]) : wave_rol1(L.rs[q][c]);
-    }
-  };
-  for (int s = 0; s < 64; ++s) step(s);
-}
-
-template <class R, int U, bool MASK>
-__device__ __forceinline__ void super_pair(Lane<R, U> &L, const float *src,
-                                           float *sacc, bool diag, int w,
-                                           int lane, float eps,
-                                           const bool (&vt)[U], int gb0src,
-                                           int n) {
-  constexpr int P = 64 * U;
-  constexpr int ST = kWaves * P;
-  // Diagonal super-tile, two measured strategies: with 8 per lane every wave
-  // meets all four tiles without reactions (16 tile passes, all waves equally
-  // long: 11.77 ms at N = 262144 against 12.01 ms the other way); with 2 or
-  // 4 per lane the six tile pairs with reactions (4 per lane: 13.13 -> 12.30
-  // ms).
-  constexpr bool kDiagReactions = U <= 4;
-  // the pass of a wave over its own tile holds the self pairs: +0 when eps^3
-  // is a normal float, masked otherwise
-  const bool self_masked = diag && !self_term_vanishes(eps);
-  if (diag && !kDiagReactions) {
-    if (self_masked)
-      tile_pass<R, U, false, true, true>(L, src, w, lane, eps, vt,
-                                         gb0src + w * P, n);
-    else
-      tile_pass<R, U, false, MASK>(L, src, w, lane, eps, vt, gb0src + w * P,
-                                   n);
-#pragma unroll 1
-    for (int b = 1; b < kWaves; ++b) {
-      const int j = (w + b) & (kWaves - 1);
-      tile_pass<R, U, false, MASK>(L, src, j, lane, eps, vt, gb0src + j * P,
-                                   n);
-    }
-    return;
-  }
-  if (diag) {
-    // Pass 0: each wave against its own tile, without reactions (self terms
-    // +0 or masked), and zeroes that tile's reaction sums.  Pass b > 0: wave w
-    // meets tile j = w + b only if j < 4, with reactions, so each of the six
-    // tile pairs is evaluated once; tile j is visited by one wave per pass.
-    // Last, each wave subtracts the negated reactions its own tile received.
-    {
-      const int o = w * P + lane * U;
-#pragma unroll
-      for (int q = 0; q < U; ++q)
-#pragma unroll
-        for (int c = 0; c < R::ACC; ++c) sacc[c * ST + o + q] = 0.0f;
-    }
-    if (self_masked)
-      tile_pass<R, U, false, true, true>(L, src, w, lane, eps, vt,
-                                         gb0src + w * P, n);
-    else
-      tile_pass<R, U, false, MASK>(L, src, w, lane, eps, vt, gb0src + w * P,
-                                   n);
-    __syncthreads();
-#pragma unroll 1
-    for (int b = 1; b < kWaves; ++b) {
-      const int j = w + b;
-      if (j < kWaves) {
-        const int o = j * P + lane * U;
-#pragma unroll
-        for (int q = 0; q < U; ++q)
-#pragma unroll
-          for (int c = 0; c < R::ACC; ++c) L.rs[q][c] = sacc[c * ST + o + q];
-        tile_pass<R, U, true, MASK>(L, src, j, lane, eps, vt, gb0src + j * P,
-                                    n);
-#pragma unroll
-        for (int q = 0; q < U; ++q)
-#pragma unroll
-          for (int c = 0; c < R::ACC; ++c) sacc[c * ST + o + q] = L.rs[q][c];
-      }
-      __syncthreads(); // tile j passes to the next wave
-    }
-    const int o = w * P + lane * U;
-#pragma unroll
-    for (int k = 0; k < U; ++k) R::sub_reaction(L.a[k], sacc + o + k, ST);
-    return;
-  }
-#pragma unroll 1
-  for (int b = 0; b < kWaves; ++b) {
-    const int j = (w + b) & (kWaves - 1);
-    // tile j's sums start at zero with its first visitor (b = 0, w = j)
-    const int o = j * P + lane * U;
-#pragma unroll
-    for (int q = 0; q < U; ++q)
-#pragma unroll
-      for (int c = 0; c < R::ACC; ++c)
-        L.rs[q][c] = b ? sacc[c * ST + o + q] : 0.0f;
-    tile_pass<R, U, true, MASK>(L, src, j, lane, eps, vt, gb0src + j * P, n);
-#pragma unroll
-    for (int q = 0; q < U; ++q)
-#pragma unroll
-      for (int c = 0; c < R::ACC; ++c) sacc[c * ST + o + q] = L.rs[q][c];
-    __syncthreads(); // tile j passes to the next wave
-  }
-}
-
-// Targets of super-tile ga held by this lane (wave w): inputs, zeroed sums
-// and validity (index < n).
-template <class R, int U>
-__device__ __forceinline__ void load_targets(Lane<R, U> &T, bool (&vt)[U],
-                                             const SymArgs &a, int ga, int w,
-                                             int lane) {
-  constexpr int P = 64 * U;
-  constexpr int ST = kWaves * P;
-  const int t0 = ga * ST + w * P + lane * U;
-#pragma unroll
-  for (int k = 0; k < U; ++k) {
-    R::load(a, t0 + k, T.t[k]);
-    vt[k] = t0 + k < a.n;
-#pragma unroll
-    for (int e = 0; e < R::ACC; ++e) T.a[k][e] = 0.0f;
-  }
-}
-
-// Super-tile pair (ga, gb), gb >= ga: stages source super-tile gb in LDS,
-// adds its terms to the targets' sums and, for gb > ga, writes the negated
-// reaction sums of its particles to sp ([ACC][ST] floats).  Called by every
-// thread of the workgroup (it contains barriers).
-template <class R, int U>
-__device__ __forceinline__ void pair_step(Lane<R, U> &T, const bool (&vt)[U],
-                                          const SymArgs &a, float *src,
-                                          float *sacc, int ga, int gb,
-                                          float *sp) {
-  constexpr int P = 64 * U;
-  constexpr int ST = kWaves * P;
-  const int tid = threadIdx.x;
-  const int w = tid >> 6, lane = tid & 63;
-  const int n = a.n;
-  __syncthreads(); // the previous super-tile and its sums are written out
-#pragma unroll
-  for (int l = 0; l < ST / 256; ++l) {
-    float v[R::SRC];
-    R::load(a, gb * ST + l * 256 + tid, v);
-    const int o = lds_slot<U>(l * 256 + tid);
-#pragma unroll
-    for (int e = 0; e < R::SRC; ++e) src[e * ST + o] = v[e];
-  }
-  __syncthreads();
-
-  // only the last super-tile holds padding particles (gb >= ga)
-  bool masked = false;
-  if constexpr (R::MASKED_TAIL) masked = (n % ST) != 0 && (gb + 1) * ST > n;
-  if (masked)
-    super_pair<R, U, R::MASKED_TAIL>(T, src, sacc, gb == ga, w, lane, a.c.eps,
-                                     vt, gb * ST, n);
-  else
-    super_pair<R, U, false>(T, src, sacc, gb == ga, w, lane, a.c.eps, vt,
-                            gb * ST, n);
-  if (gb == ga) return;
-#pragma unroll
-  for (int l = 0; l < R::ACC * ST / 256; ++l)
-    sp[l * 256 + tid] = sacc[l * 256 + tid];
-}
-
-// The targets' sums as one row partial ([ACC][ST] floats at fp).
-template <class R, int U>
-__device__ __forceinline__ void store_row(const Lane<R, U> &T, float *fp,
-                                          int w, int lane) {
-  constexpr int P = 64 * U;
-  constexpr int ST = kWaves * P;
-  float *q = fp + w * P + lane * U;
-#pragma unroll
-  for (int k = 0; k < U; ++k)
-#pragma unroll
-    for (int e = 0; e < R::ACC; ++e) q[e * ST + k] = T.a[k][e];
-}
 
 // f += partial(0), partial(1), ... in that order (SUB: f -= ...), with
 // kInFlight partials loaded ahead of the running sum: the loads do not
@@ -783,19 +453,24 @@ __device__ __forceinline__ bool combine_runs(float (&f)[R::ACC],
   }
 }
 
-// ---- row form: one wave holds a whole row super-tile ------------------------
+// ---- pair kernels: a wave holds a whole row ---------------------------------
 //
-// Super-tiles of ST = 64 U particles, U targets per lane: each wave of the
-// workgroup holds all targets of the row super-tile GA and takes its share of
-// the source super-tile GB in sets of 64 sources, one source per lane and
-// step.  Per step a lane reads one source (SRC floats) from LDS and rotates
-// ACC reaction sums for U pair terms; no barrier inside a super-tile pair.
-//   * U >= 4: wave w meets sets w, w + 4, .. of GB (U / 4 of them) and writes
-//     their reaction sums;  U = 2: two waves share a set, each half of its 64
-//     steps, and add their reaction sums through LDS;
-//   * at the end of the work item the four waves' target sums are added in a
-//     fixed tree, (0 + 2) + (1 + 3), and written as one row partial.
-// Partials and finalize are those of the four-wave form with the same ST.
+// Super-tiles of ST = 64 U M particles: M rows of 64 U, U targets per lane.
+// Each wave of the workgroup holds the same row of the super-tile GA (every
+// wave all its targets) and takes its share of the source super-tile GB in
+// sets of 64 sources, one source per lane and step.  Per step a lane reads
+// one source (SRC floats) from LDS and rotates ACC reaction sums for U pair
+// terms; no barrier inside a row.
+//   * U = 8 or 4: wave w meets sets w, w + 4, .. of GB;  U = 2: two waves
+//     share a set, each half of its 64 steps, and add their reaction sums
+//     through LDS;
+//   * at the end of a row the waves' target sums are added in a fixed tree,
+//     (0 + 2) + (1 + 3);
+//   * M = 1: the row meets every GB of the work item before that;  M > 1: the
+//     rows of GA meet one GB in turn, and the reaction sums of a set, owned by
+//     one wave, wait in LDS from row to row (one reaction partial per ST x ST
+//     pairs, 1 / M of M = 1's).  M = 4 runs 8 waves per workgroup: half as
+//     long items, a shorter last round for the same partials.
 // The sources lie twice in LDS (128 floats per coordinate and wave), so that
 // step s reads at lane + s with no wrap, its offset in the instruction.
 //
@@ -804,18 +479,30 @@ __device__ __forceinline__ bool combine_runs(float (&f)[R::ACC],
 // for the adjoint); with 8 x 1 it is 3 and 3 for 8.  In the pair loop alone,
 // sustained at 4 waves per SIMD, SIMD cycles (at 2.4 GHz) per wave pair term
 // 2 x 2 -> 8 x 1: forward 56 -> 47, adjoint 85 -> 72, fused 120 -> 94, Kahan
-// 102 -> 89.
-template <class R, int U>
+// 102 -> 89.  8 x 8 in four-wave passes with a barrier per pass: 50 (3 waves
+// per SIMD, 48 KiB of LDS).
+template <class R, int U, int M = 1>
 struct RowShape {
   static_assert(U == 2 || U == 4 || U == 8, "targets per lane");
-  static constexpr int ST = 64 * U;                  // super-tile
+  static_assert(M == 1 || U == 8, "rows per super-tile");
+  static constexpr int RT = 64 * U;                  // row
+  static constexpr int ST = RT * M;                  // super-tile
+  static constexpr int W = M > 2 ? 8 : 4;            // waves per workgroup
+  static constexpr int SETS = ST / 64;               // source sets
   static constexpr int PARTS = U >= 4 ? 1 : 4 / U;   // waves per set
   static constexpr int STEPS = 64 / PARTS;           // steps of a wave per set
-  static constexpr int SRC_FLOATS = kWaves * R::SRC * 128;
-  static constexpr int REACT_FLOATS = PARTS > 1 ? kWaves * R::ACC * 64 : 0;
-  static constexpr int SUM_FLOATS = 2 * R::ACC * ST; // the tree's two buffers
-  static constexpr int LDS_FLOATS = SRC_FLOATS + REACT_FLOATS > SUM_FLOATS
-                                        ? SRC_FLOATS + REACT_FLOATS
+  // LDS: the waves' sources, and in the same place (a barrier between) the
+  // two buffers of the tree; then the reaction sums that wait or meet there
+  static constexpr int SRC_FLOATS = W * R::SRC * 128;
+  static constexpr int SUM_FLOATS = W / 2 * R::ACC * RT;
+  static constexpr int REACT = PARTS == 1 && SUM_FLOATS > SRC_FLOATS
+                                   ? SUM_FLOATS
+                                   : SRC_FLOATS;
+  static constexpr int REACT_FLOATS = PARTS > 1 ? W * R::ACC * 64
+                                      : M > 1   ? R::ACC * ST
+                                                : 0;
+  static constexpr int LDS_FLOATS = REACT + REACT_FLOATS > SUM_FLOATS
+                                        ? REACT + REACT_FLOATS
                                         : SUM_FLOATS;
 };
 
@@ -830,9 +517,9 @@ __device__ __forceinline__ void wave_lds_fence() {
 
 // Steps [s0, s0 + STEPS) of the wave's targets t against the 64 sources at
 // src ([SRC][128]): target sums into a, reaction sums of source (lane + s1)
-// mod 64 into rs.  masked: sources at or past index n - src0 and, in the set
-// of the wave's own targets self (-1: another set), the self pairs (step 0)
-// contribute nothing.
+// mod 64 into rs.  masked: sources at or past index `valid` of the set and,
+// in the set of the wave's own targets self (-1: another set), the self pairs
+// (step 0) contribute nothing.
 template <class R, int U>
 __device__ __forceinline__ void
 row_pass(const float (&t)[U][R::SRC], float (&a)[U][R::ACC],
@@ -859,40 +546,45 @@ row_pass(const float (&t)[U][R::SRC], float (&a)[U][R::ACC],
       const bool vs = ((lane + s0 + s) & 63) < valid;
 #pragma unroll
       for (int k = 0; k < U; ++k)
-        R::template pair<true, true>(sv, t[k], a[k], rs, eps,
-                                     vs && !(k == self && s0 + s == 0));
+        R::pair_masked(sv, t[k], a[k], rs, eps,
+                       vs && !(k == self && s0 + s == 0));
 #pragma unroll
       for (int e = 0; e < R::ACC; ++e) rs[e] = lds_rol1(rs[e]);
     }
   }
 }
 
-// Work item: row super-tile ga against source super-tiles [gb0, gb1), gb0 >=
-// ga.  Row partial ([ACC][ST]) to fp, the (negated) reaction sums of gb > ga
-// to sp_at(gb) ([ACC][ST]).  lds: LDS_FLOATS.  Called by every thread of the
-// workgroup.  The diagonal (gb == ga) is met whole, without reactions.
-template <class R, int U, class SpAt>
-__device__ __forceinline__ void row_item(const SymArgs &a, float *lds, int ga,
-                                         int gb0, int gb1, float *fp,
-                                         SpAt sp_at) {
-  using S = RowShape<R, U>;
+// Row `row` of super-tile ga (targets ga * ST + row * RT ..) against source
+// super-tiles [gb0, gb1), gb0 >= ga: the wave's target sums into sum, the
+// (negated) reaction sums of gb > ga after the last row to sp_at(gb)
+// ([ACC][ST]).  lds: LDS_FLOATS.  Called by every thread of the workgroup.
+// On the diagonal (gb == ga) a row meets its own sets without reactions (each
+// of their pairs twice) and, M > 1, those of the rows after it with; their
+// reaction sums wait for those rows in LDS (add_waves subtracts them).
+template <class R, int U, int M, class SpAt>
+__device__ __forceinline__ void meet_sources(float (&sum)[U][R::ACC],
+                                             const SymArgs &a, float *lds,
+                                             int ga, int row, int gb0, int gb1,
+                                             SpAt sp_at) {
+  using S = RowShape<R, U, M>;
   constexpr int ST = S::ST;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int part = w % S::PARTS, first = w / S::PARTS;
   const int s0 = part * S::STEPS;
-  float t[U][R::SRC], sum[U][R::ACC];
+  float t[U][R::SRC];
 #pragma unroll
   for (int k = 0; k < U; ++k) {
-    R::load(a, ga * ST + k * 64 + lane, t[k]);
+    R::load(a, ga * ST + row * S::RT + k * 64 + lane, t[k]);
 #pragma unroll
     for (int e = 0; e < R::ACC; ++e) sum[k][e] = 0.0f;
   }
   float *src = lds + w * (R::SRC * 128);
-  float *react = lds + S::SRC_FLOATS;
+  float *react = lds + S::REACT;
   const bool self_vanishes = self_term_vanishes(a.c.eps);
   float nxt[R::SRC]; // the next set's sources, in flight during a pass
-  R::load(a, gb0 * ST + first * 64 + lane, nxt);
-  int gb = gb0, q = first;
+  // the diagonal's sets before the row met it there already
+  int gb = gb0, q = (M > 1 && gb0 == ga ? row * U : 0) + first;
+  R::load(a, gb * ST + q * 64 + lane, nxt);
   while (gb < gb1) {
     wave_lds_fence();
 #pragma unroll
@@ -902,8 +594,8 @@ __device__ __forceinline__ void row_item(const SymArgs &a, float *lds, int ga,
     }
     wave_lds_fence();
     const int g = gb, set = q;
-    q += kWaves;
-    if (q >= U) {
+    q += S::W / S::PARTS;
+    if (q >= S::SETS) {
       q = first;
       ++gb;
     }
@@ -912,17 +604,22 @@ __device__ __forceinline__ void row_item(const SymArgs &a, float *lds, int ga,
     const int left = a.n - (g * ST + set * 64); // sources before the padding
     bool masked = g == ga && !self_vanishes;
     if constexpr (R::MASKED_TAIL) masked = masked || left < 64;
+    float *held = react + set * 64 + lane; // M > 1: this wave's, row to row
     float rs[R::ACC];
 #pragma unroll
     for (int e = 0; e < R::ACC; ++e) rs[e] = 0.0f;
+    // (a diagonal set's first visitor is row 0, but its own row's sums are
+    // not kept)
+    if (M > 1 && row > 0) R::fetch(rs, held, ST);
     if (left > 0) // the same for the waves that share a set
       row_pass<R, U>(t, sum, rs, src, lane, s0, a.c.eps, masked,
-                     g == ga ? set : -1, left);
-    if (g == ga) continue;
-    float *sp = sp_at(g) + set * 64;
+                     g == ga ? set - row * U : -1, left);
+    if (g == ga && (M == 1 || set < (row + 1) * U)) continue;
     if constexpr (S::PARTS == 1) {
+      const bool out = M == 1 || (row == M - 1 && g > ga);
+      float *sp = out ? sp_at(g) + set * 64 + lane : held;
 #pragma unroll
-      for (int e = 0; e < R::ACC; ++e) sp[e * ST + lane] = rs[e];
+      for (int e = 0; e < R::ACC; ++e) sp[e * ST] = rs[e];
     } else {
       // lane l holds the sums of source (l + s1) mod 64
       const int m = (lane + s0 + S::STEPS) & 63;
@@ -938,49 +635,110 @@ __device__ __forceinline__ void row_item(const SymArgs &a, float *lds, int ga,
           R::fetch(v, react + (w + p) * R::ACC * 64 + lane, 64);
           R::add_v(f, v);
         }
+        float *sp = sp_at(g) + set * 64 + lane;
 #pragma unroll
-        for (int e = 0; e < R::ACC; ++e) sp[e * ST + lane] = f[e];
+        for (int e = 0; e < R::ACC; ++e) sp[e * ST] = f[e];
       }
       __syncthreads(); // read before the next pair overwrites it
     }
   }
+}
 
-  // target sums of the four waves: (0 + 2) + (1 + 3); waves 0 and 1 each
-  // finish half of the targets
-  auto put = [&](int slot, int k0, int k1) {
+// The W waves' target sums, halves added until two are left, to fp ([ACC][RT],
+// one coordinate `stride` apart), added to what it holds with ADD.  Waves 0
+// and 1 each finish half of the targets and subtract the row's reaction sums
+// from its own super-tile (held: [ACC][stride]; nullptr: none).  Leaves the
+// LDS free for reuse.
+template <class R, int U, int W, bool ADD>
+__device__ __forceinline__ void add_waves(float (&sum)[U][R::ACC], float *lds,
+                                          const float *held, float *fp,
+                                          int stride) {
+  constexpr int RT = 64 * U;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // buffer b of the tree ([ACC][RT])
+  auto buf = [&](int b) { return lds + b * (R::ACC * RT) + lane; };
+  // (the scheduling barriers keep one target's values in flight, not all U:
+  // registers here would cost the pair loop its waves)
+  auto put = [&](float *p, int k0, int k1) {
 #pragma unroll
     for (int k = 0; k < U; ++k)
       if (k >= k0 && k < k1)
 #pragma unroll
-        for (int e = 0; e < R::ACC; ++e)
-          lds[(slot * R::ACC + e) * ST + k * 64 + lane] = sum[k][e];
+        for (int e = 0; e < R::ACC; ++e) p[e * RT + k * 64] = sum[k][e];
   };
-  auto take = [&](int slot, int k0, int k1) {
+  auto take = [&](const float *p, int k0, int k1) {
 #pragma unroll
     for (int k = 0; k < U; ++k)
       if (k >= k0 && k < k1) {
         float v[R::ACC];
-        R::fetch(v, lds + slot * (R::ACC * ST) + k * 64 + lane, ST);
+        R::fetch(v, p + k * 64, RT);
         R::add_v(sum[k], v);
+        __builtin_amdgcn_sched_barrier(0);
       }
   };
   __syncthreads(); // every wave is done with its sources
-  if (w >= 2) put(w - 2, 0, U);
+#pragma unroll
+  for (int h = W / 2; h >= 2; h >>= 1) {
+    if (w >= h && w < 2 * h) put(buf(w & (h - 1)), 0, U);
+    __syncthreads();
+    if (w < h) take(buf(w & (h - 1)), 0, U);
+    __syncthreads();
+  }
+  if (w == 0) put(buf(0), U / 2, U);
+  if (w == 1) put(buf(1), 0, U / 2);
   __syncthreads();
-  if (w < 2) take(w, 0, U);
-  __syncthreads();
-  if (w == 0) put(0, U / 2, U);
-  if (w == 1) put(1, 0, U / 2);
-  __syncthreads();
-  if (w >= 2) return;
-  if (w == 0) take(1, 0, U / 2);
-  else take(0, U / 2, U);
+  if (w == 0) take(buf(1), 0, U / 2);
+  if (w == 1) take(buf(0), U / 2, U);
 #pragma unroll
   for (int k = 0; k < U; ++k)
-    if ((k < U / 2) == (w == 0))
+    if (w == (k < U / 2 ? 0 : 1)) {
+      float *p = fp + k * 64 + lane;
+      if (held) {
+        float v[R::ACC];
+        R::fetch(v, held + k * 64 + lane, stride);
+        R::sub_v(sum[k], v);
+      }
+      if constexpr (ADD) {
+        float v[R::ACC];
+        R::fetch(v, p, stride);
+        R::add_v(v, sum[k]);
 #pragma unroll
-      for (int e = 0; e < R::ACC; ++e)
-        fp[e * ST + k * 64 + lane] = sum[k][e];
+        for (int e = 0; e < R::ACC; ++e) p[e * stride] = v[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < R::ACC; ++e) p[e * stride] = sum[k][e];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  __syncthreads();
+}
+
+// Work item: super-tile ga against source super-tiles [gb0, gb1), gb0 >= ga.
+// Row partial ([ACC][ST]) to fp, reaction sums to sp_at(gb) ([ACC][ST]).
+template <class R, int U, int M, class SpAt>
+__device__ __forceinline__ void row_item(const SymArgs &a, float *lds, int ga,
+                                         int gb0, int gb1, float *fp,
+                                         SpAt sp_at) {
+  using S = RowShape<R, U, M>;
+  float sum[U][R::ACC];
+  if constexpr (M == 1) {
+    meet_sources<R, U, M>(sum, a, lds, ga, 0, gb0, gb1, sp_at);
+    add_waves<R, U, S::W, false>(sum, lds, nullptr, fp, S::ST);
+  } else {
+#pragma unroll 1
+    for (int gb = gb0; gb < gb1; ++gb)
+#pragma unroll 1
+      for (int row = 0; row < M; ++row) {
+        // rows of padding only: the last super-tile's, which has no reactions
+        if (ga * S::ST + row * S::RT >= a.n) break;
+        meet_sources<R, U, M>(sum, a, lds, ga, row, gb, gb + 1, sp_at);
+        const float *held =
+            gb == ga && row > 0 ? lds + S::REACT + row * S::RT : nullptr;
+        float *f = fp + row * S::RT;
+        if (gb == gb0) add_waves<R, U, S::W, false>(sum, lds, held, f, S::ST);
+        else add_waves<R, U, S::W, true>(sum, lds, held, f, S::ST);
+      }
+  }
 }
 
 // Work item -> (row ga, chunk c): rows are enumerated in order, row ga
@@ -995,44 +753,40 @@ __device__ __forceinline__ int item_row(long long it, int ts, int L) {
   return lo;
 }
 
-template <class R, int U>
-__global__ __launch_bounds__(256) void sym_row_kernel(SymArgs a) {
-  __shared__ float lds[RowShape<R, U>::LDS_FLOATS];
-  constexpr int ST = RowShape<R, U>::ST;
-  const int ts = a.ts, L = a.chunk;
-  const long long it = blockIdx.x;
-  const int ga = item_row(it, ts, L);
-  const int gb0 = ga + (int)(it - row_first(ga, ts, L)) * L;
-  row_item<R, U>(a, lds, ga, gb0, min(gb0 + L, ts),
-                 a.fpart + (size_t)it * (R::ACC * ST), [&](int gb) {
-                   return a.spart + (size_t)pair_slot(ga, gb, ts) * (R::ACC * ST);
-                 });
+// Work item of a launch -> super-tile ga, its chunk c (row partial
+// row_first(ga) + c).  With one super-tile per item the diagonal pairs, the
+// shorter ones, come last: they fill the last round.
+__device__ __forceinline__ void sym_item(long long it, int ts, int L, int &ga,
+                                         int &c) {
+  if (L == 1) {
+    const long long pairs = (long long)ts * (ts - 1) / 2;
+    if (it >= pairs) {
+      ga = (int)(it - pairs);
+      c = 0;
+    } else { // rows of lengths ts - 1, .. 1
+      ga = item_row(it, ts - 1, 1);
+      c = (int)(it - row_first(ga, ts - 1, 1)) + 1;
+    }
+  } else {
+    ga = item_row(it, ts, L);
+    c = (int)(it - row_first(ga, ts, L));
+  }
 }
 
-template <class R, int U>
-__global__ __launch_bounds__(256) void sym_kernel(SymArgs a) {
-  constexpr int P = 64 * U;
-  constexpr int ST = kWaves * P;
-  __shared__ float4 src4[R::SRC][ST / 4];  // source super-tile, SoA
-  __shared__ float4 sacc4[R::ACC][ST / 4]; // reaction sums of its 4 tiles
-  float *src = reinterpret_cast<float *>(src4);
-  float *sacc = reinterpret_cast<float *>(sacc4);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+template <class R, int U, int M>
+__global__ __launch_bounds__((64 * RowShape<R, U, M>::W)) void sym_kernel(SymArgs a) {
+  __shared__ float lds[RowShape<R, U, M>::LDS_FLOATS];
+  constexpr int ST = RowShape<R, U, M>::ST;
   const int ts = a.ts, L = a.chunk;
-  const long long it = blockIdx.x;
-  const int ga = item_row(it, ts, L);
-  const int c = (int)(it - row_first(ga, ts, L));
+  int ga, c;
+  sym_item(blockIdx.x, ts, L, ga, c);
   const int gb0 = ga + c * L;
-  const int gb1 = min(gb0 + L, ts);
-
-  Lane<R, U> T;
-  bool vt[U];
-  load_targets(T, vt, a, ga, w, lane);
-  for (int gb = gb0; gb < gb1; ++gb)
-    pair_step(T, vt, a, src, sacc, ga, gb,
-              gb > ga ? a.spart + (size_t)pair_slot(ga, gb, ts) * (R::ACC * ST)
-                      : nullptr);
-  store_row(T, a.fpart + (size_t)it * (R::ACC * ST), w, lane);
+  row_item<R, U, M>(
+      a, lds, ga, gb0, min(gb0 + L, ts),
+      a.fpart + (size_t)(row_first(ga, ts, L) + c) * (R::ACC * ST),
+      [&](int gb) {
+        return a.spart + (size_t)pair_slot(ga, gb, ts) * (R::ACC * ST);
+      });
 }
 
 constexpr int kTileRuns = 4; // runs per particle, tile-pair finalize
@@ -1108,45 +862,19 @@ __device__ __forceinline__ void band_item(long long it, int b0, int W, int L,
   }
 }
 
-template <class R, int U>
-__global__ __launch_bounds__(256) void sym_band_kernel(SymArgs a) {
-  constexpr int P = 64 * U;
-  constexpr int ST = kWaves * P;
-  __shared__ float4 src4[R::SRC][ST / 4];
-  __shared__ float4 sacc4[R::ACC][ST / 4];
-  float *src = reinterpret_cast<float *>(src4);
-  float *sacc = reinterpret_cast<float *>(sacc4);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+template <class R, int U, int M>
+__global__ __launch_bounds__((64 * RowShape<R, U, M>::W)) void sym_band_kernel(SymArgs a) {
+  __shared__ float lds[RowShape<R, U, M>::LDS_FLOATS];
+  constexpr int ST = RowShape<R, U, M>::ST;
   const int L = a.chunk, b0 = a.b0, W = a.bw;
   const long long it = blockIdx.x;
   int ga, gb0;
   band_item(it, b0, W, L, ga, gb0);
-  const int gb1 = min(gb0 + L, b0 + W);
-  Lane<R, U> T;
-  bool vt[U];
-  load_targets(T, vt, a, ga, w, lane);
-  for (int gb = gb0; gb < gb1; ++gb)
-    pair_step(T, vt, a, src, sacc, ga, gb,
-              gb > ga ? a.spart + (size_t)band_pair_slot(ga, gb, b0, W) *
-                                      (R::ACC * ST)
-                      : nullptr);
-  store_row(T, a.fpart + (size_t)it * (R::ACC * ST), w, lane);
-}
-
-// The same in the row form (U targets per lane, ST = 64 U).
-template <class R, int U>
-__global__ __launch_bounds__(256) void sym_row_band_kernel(SymArgs a) {
-  __shared__ float lds[RowShape<R, U>::LDS_FLOATS];
-  constexpr int ST = RowShape<R, U>::ST;
-  const int L = a.chunk, b0 = a.b0, W = a.bw;
-  const long long it = blockIdx.x;
-  int ga, gb0;
-  band_item(it, b0, W, L, ga, gb0);
-  row_item<R, U>(a, lds, ga, gb0, min(gb0 + L, b0 + W),
-                 a.fpart + (size_t)it * (R::ACC * ST), [&](int gb) {
-                   return a.spart + (size_t)band_pair_slot(ga, gb, b0, W) *
-                                        (R::ACC * ST);
-                 });
+  row_item<R, U, M>(
+      a, lds, ga, gb0, min(gb0 + L, b0 + W),
+      a.fpart + (size_t)it * (R::ACC * ST), [&](int gb) {
+        return a.spart + (size_t)band_pair_slot(ga, gb, b0, W) * (R::ACC * ST);
+      });
 }
 
 // Per particle: its band rows (chunk order) minus its band reactions (GA
@@ -1274,48 +1002,21 @@ __device__ __forceinline__ void leave_queue(const SymBatchArgs &b) {
   }
 }
 
-template <int U>
-__global__ __launch_bounds__(256) void sym_batch_kernel(SymBatchArgs b) {
+template <int U, int M>
+__global__
+__launch_bounds__((64 * RowShape<ForceRule, U, M>::W), 4) void sym_batch_kernel(SymBatchArgs b) {
   using R = ForceRule;
-  constexpr int P = 64 * U;
-  constexpr int ST = kWaves * P;
-  __shared__ float4 src4[R::SRC][ST / 4];
-  __shared__ float4 sacc4[R::ACC][ST / 4];
+  constexpr int ST = RowShape<R, U, M>::ST;
+  __shared__ float lds[RowShape<R, U, M>::LDS_FLOATS];
   __shared__ int s_item;
-  float *src = reinterpret_cast<float *>(src4);
-  float *sacc = reinterpret_cast<float *>(sacc4);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (;;) {
     const int item = next_item(b, &s_item);
     if (item >= b.num_items) break;
     const int4 it = b.items[item];
     const SymArgs a = system_view(b, it.x, ST);
     float *slot = b.part + (size_t)it.w * (2 * R::ACC * ST);
-    Lane<R, U> T;
-    bool vt[U];
-    load_targets(T, vt, a, it.y, w, lane);
-    pair_step(T, vt, a, src, sacc, it.y, it.z, slot + R::ACC * ST);
-    store_row(T, slot, w, lane);
-  }
-  leave_queue(b);
-}
-
-// The same in the row form (U targets per lane, ST = 64 U).
-template <int U>
-__global__ __launch_bounds__(256, 4) void sym_row_batch_kernel(SymBatchArgs b) {
-  using R = ForceRule;
-  constexpr int ST = RowShape<R, U>::ST;
-  __shared__ float lds[RowShape<R, U>::LDS_FLOATS];
-  __shared__ int s_item;
-  for (;;) {
-    // its barriers also hold the item's LDS until every wave is done with it
-    const int item = next_item(b, &s_item);
-    if (item >= b.num_items) break;
-    const int4 it = b.items[item];
-    const SymArgs a = system_view(b, it.x, ST);
-    float *slot = b.part + (size_t)it.w * (2 * R::ACC * ST);
-    row_item<R, U>(a, lds, it.y, it.z, it.z + 1, slot,
-                   [&](int) { return slot + R::ACC * ST; });
+    row_item<R, U, M>(a, lds, it.y, it.z, it.z + 1, slot,
+                      [&](int) { return slot + R::ACC * ST; });
   }
   leave_queue(b);
 }
@@ -1356,18 +1057,15 @@ using KernelFn = void (*)(SymArgs);
 // Kernels of one launch shape and its super-tile.  runs: finalize runs per
 // particle.
 struct SymShape {
-  int st, runs;
+  int st, threads, runs;
   KernelFn pairs, finalize;
 };
 
-template <class R, int U, int RUNS>
-constexpr SymShape row_shape() {
-  return {64 * U, RUNS, sym_row_kernel<R, U>, sym_finalize<R, 64 * U, RUNS>};
-}
-
-template <class R, int U>
-constexpr SymShape wave_shape() {
-  return {256 * U, 1, sym_kernel<R, U>, sym_finalize<R, 256 * U, 1>};
+template <class R, int U, int M, int RUNS>
+constexpr SymShape sym_shape() {
+  constexpr int ST = 64 * U * M;
+  return {ST, 64 * RowShape<R, U, M>::W, RUNS, sym_kernel<R, U, M>,
+          sym_finalize<R, ST, RUNS>};
 }
 
 // Targets per lane of a tile-pair shape: `unroll` particles per lane and
@@ -1378,23 +1076,23 @@ int tile_targets(int unroll, int items) {
   return unroll == 2 && items == 1 ? 4 : unroll;
 }
 
-// Super-tiles of 512 (2 per lane) run in the row form, larger ones in the
-// four-wave form; tile pairs in the row form with one super-tile per tile or
-// pair of tiles.
+// Super-tile shapes: M = unroll / 2 rows of 512.  Tile pairs: one row per
+// super-tile, of one tile or a pair of tiles.
 template <class R>
 const SymShape *find_shape(int unroll, bool tiles, int items) {
-  static const SymShape row2 = row_shape<R, 2, kTileRuns>(),
-                        row4 = row_shape<R, 4, kTileRuns>(),
-                        row8 = row_shape<R, 8, 1>(), wave4 = wave_shape<R, 4>();
+  static const SymShape tile2 = sym_shape<R, 2, 1, kTileRuns>(),
+                        tile4 = sym_shape<R, 4, 1, kTileRuns>(),
+                        rows1 = sym_shape<R, 8, 1, 1>(),
+                        rows2 = sym_shape<R, 8, 2, 1>();
   if (tiles) {
     if (unroll != 2 && unroll != 4) return nullptr;
-    return tile_targets(unroll, items) == 2 ? &row2 : &row4;
+    return tile_targets(unroll, items) == 2 ? &tile2 : &tile4;
   }
-  if (unroll == 2) return &row8;
-  if (unroll == 4) return &wave4;
-  if constexpr (R::WAVE8) {
-    static const SymShape wave8 = wave_shape<R, 8>();
-    if (unroll == 8) return &wave8;
+  if (unroll == 2) return &rows1;
+  if (unroll == 4) return &rows2;
+  if constexpr (R::ROWS4) {
+    static const SymShape rows4 = sym_shape<R, 8, 4, 1>();
+    if (unroll == 8) return &rows4;
   }
   return nullptr;
 }
@@ -1408,23 +1106,24 @@ bool sym_banded(int unroll, bool tiles, int chunk, int acc, size_t n) {
 }
 
 struct BandShape {
-  int unroll, st;
+  int unroll, st, threads;
   KernelFn pairs, fold, finish;
 };
 
-// Band kernels of rule R: 2 (row form), 4 or 8 particles per lane (Kahan: 2
-// or 4).
+// Band kernels of rule R: 2, 4 or 8 particles per lane (Kahan: 2 or 4).
+template <class R, int M>
+constexpr BandShape band_shape() {
+  return {2 * M, 512 * M, 64 * RowShape<R, 8, M>::W, sym_band_kernel<R, 8, M>,
+          sym_band_fold<R, 512 * M>, sym_band_finish<R>};
+}
+
 template <class R>
 const BandShape *find_band_shape(int unroll) {
-  static const BandShape b2 = {2, 512, sym_row_band_kernel<R, 8>,
-                               sym_band_fold<R, 512>, sym_band_finish<R>},
-                         b4 = {4, 1024, sym_band_kernel<R, 4>,
-                               sym_band_fold<R, 1024>, sym_band_finish<R>};
+  static const BandShape b2 = band_shape<R, 1>(), b4 = band_shape<R, 2>();
   if (unroll == 2) return &b2;
   if (unroll == 4) return &b4;
-  if constexpr (R::WAVE8) {
-    static const BandShape b8 = {8, 2048, sym_band_kernel<R, 8>,
-                                 sym_band_fold<R, 2048>, sym_band_finish<R>};
+  if constexpr (R::ROWS4) {
+    static const BandShape b8 = band_shape<R, 4>();
     if (unroll == 8) return &b8;
   }
   return nullptr;
@@ -1439,7 +1138,7 @@ struct BandPlan {
 };
 
 BandPlan band_plan(size_t n, int unroll, int chunk) {
-  const int st = kWaves * 64 * unroll;
+  const int st = 256 * unroll;
   const int ts = (int)((n + st - 1) / st);
   const size_t per_slot = sizeof(float) * 3 * st;
   for (int w = ts; w >= 1; --w) {
@@ -1476,7 +1175,8 @@ int launch_sym_banded(const BandShape *band, SymArgs &a, int chunk, int n,
     const long long items = band_items(a.b0, a.bw, chunk);
     int r = hip_check(
         hipLaunchKernel(reinterpret_cast<const void *>(band->pairs),
-                        dim3((unsigned)items), block, args, 0, stream),
+                        dim3((unsigned)items), dim3(band->threads), args, 0,
+                        stream),
         "symmetric band launch");
     if (!r)
       r = hip_check(hipLaunchKernel(reinterpret_cast<const void *>(band->fold),
@@ -1529,8 +1229,8 @@ int launch_sym(const SymShape *sh, SymArgs &a, int unroll, int chunk, int n,
   a.n = n;
   void *args[] = {&a};
   int r = hip_check(hipLaunchKernel(reinterpret_cast<const void *>(sh->pairs),
-                                    dim3((unsigned)blocks), dim3(256), args, 0,
-                                    stream),
+                                    dim3((unsigned)blocks), dim3(sh->threads),
+                                    args, 0, stream),
                     "symmetric pair launch");
   if (r) return r;
   const int per_block = 256 / sh->runs;
@@ -1561,12 +1261,12 @@ size_t sym_scratch_bytes(int unroll, int chunk, size_t n, int acc,
     const BandPlan bp = band_plan(n, unroll, chunk);
     if (bp.w < 1) return 0;
     return sizeof(float) * ((size_t)(bp.rows + bp.reacs) * acc *
-                                (size_t)(kWaves * 64 * unroll) +
+                                (size_t)(256 * unroll) +
                             (size_t)acc * n);
   }
   if (n == 0 || n > sym_max_particles(unroll, tiles, chunk, acc) || chunk < 1)
     return 0;
-  const long long st = (long long)kWaves * 64 * unroll;
+  const long long st = (long long)256 * unroll;
   const long long ts = ((long long)n + st - 1) / st;
   const long long slots = items_upto(ts, chunk) + ts * (ts - 1) / 2;
   return sizeof(float) * (size_t)slots * acc * (size_t)st;
@@ -1577,7 +1277,7 @@ int sym_batch_layout(int unroll, const int *sys_off, int num_systems,
                      size_t &part_bytes) {
   if (unroll != 2 && unroll != 4 && unroll != 8)
     return set_error(NB_ERR_UNSUPPORTED, "no symmetric batch kernel for shape");
-  const int ST = kWaves * 64 * unroll;
+  const int ST = 256 * unroll;
   std::vector<int4> off_diag, diag;
   sys_slot.assign(num_systems + 1, 0);
   long long slots = 0;
@@ -1604,15 +1304,17 @@ int sym_batch_layout(int unroll, const int *sys_off, int num_systems,
 
 namespace {
 template <int U> const void *batch_pairs_fn() {
-  if constexpr (U == 2)
-    return reinterpret_cast<const void *>(sym_row_batch_kernel<8>);
-  else
-    return reinterpret_cast<const void *>(sym_batch_kernel<U>);
+  return reinterpret_cast<const void *>(sym_batch_kernel<8, U / 2>);
 }
 template <int U> const void *batch_finalize_fn() {
-  return reinterpret_cast<const void *>(sym_batch_finalize<kWaves * 64 * U>);
+  return reinterpret_cast<const void *>(sym_batch_finalize<256 * U>);
 }
 } // namespace
+
+int sym_batch_threads(int unroll) {
+  return 64 * (unroll == 8 ? RowShape<ForceRule, 8, 4>::W
+                           : RowShape<ForceRule, 8, 1>::W);
+}
 
 const void *sym_batch_kernel_fn(int unroll) {
   switch (unroll) {
@@ -1652,7 +1354,8 @@ int launch_sym_batch(int unroll, const SymBatchLaunch &L, hipStream_t stream) {
   b.total = L.total;
   b.counters = L.counters;
   void *args[] = {&b};
-  int r = hip_check(hipLaunchKernel(pairs, dim3(L.grid), dim3(256), args, 0,
+  int r = hip_check(hipLaunchKernel(pairs, dim3(L.grid),
+                                    dim3(sym_batch_threads(unroll)), args, 0,
                                     stream),
                     "symmetric batch launch");
   if (r) return r;
