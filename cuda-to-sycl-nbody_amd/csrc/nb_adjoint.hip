@@ -315,22 +315,22 @@ int adjoint_config_count() { return kNumAdj; }
 const FwdConfig &adjoint_config(int cfg) { return kAdjConfigs[cfg]; }
 
 int adjoint_default_config(size_t n, bool skip) {
-  // Measured on MI355X (disk ICs), adjoint / fused us.  Tile pairs, 2 per
-  // lane: n = 4096 28.7 / 35.7, 16384 124.5 / 146.3 (super-tile pairs, 2 per
-  // lane: 141.7 / 181.0), 25600 245.8 / 289.7 (217.0 / 282.2), 32768 379.9 /
-  // 449.9.  Super-tile pairs, 2 per lane, 1 / 2 per item: 32768 354.7 / 471.7 vs
-  // 403.2 / 542.8, 65536 1219 / 1644 (tile pairs 1447 / 1771), 131072
-  // 4780 / 6511 vs 4779 / 6478, 262144 19280 / 25892 vs 19168 / 25601
-  // (4 per lane 23660 / 31135, 8 per lane 24283 / 34040).  Best
-  // target-sharded: 8192 65.8 / 74.2, 262144 38.7 / 43.5 ms.  Past 2^18 two
-  // per lane need four super-tiles per item and bands of source super-tiles
-  // (4 per lane at 2^21: 1501 / 1986 ms).
+  // Measured on MI355X (disk ICs), adjoint / fused us (device time).  Tile
+  // pairs, 2 per lane: n = 64 7.3 / 8.6 (target-sharded 256 x 1 split 2 7.1 /
+  // 8.1), 300 8.9 / 10.5 (20.7 / 23.9), 4097 17 / 21 (63 / 72), 12000 57 / 76
+  // (super-tiles of 512, 1 per item 71 / 89), 24000 162 / 215 (176 / 229),
+  // 30720 264.1 / 350.4 (274.5 / 359.1), 34000 321.8 / 428.6 (313.3 / 407.4).
+  // Super-tiles of 512, 1 / 2 per item: 65536 1041 / 1369 vs 1052 / 1411 (tile pairs 1099 / 1490), 100000 2371 / 3160 vs
+  // 2360 / 3124, 262144 16154 / 21434 vs 15812 / 21092 (super-tiles of 1024:
+  // 16461 / 22713 on a card where 2 per item took 16509 / 21775).  Best
+  // target-sharded at 262144 31.5 / 39.0 ms.  Past 2^18 four super-tiles per
+  // item and bands of source super-tiles.
   if (n <= kSymBandedMaxParticles && n > kSymSmallMaxParticles)
     return 22; // super-tile pairs, 2 per lane, 4 per item, in bands
   if (n <= kSymMaxParticles) { // skip or not: self pairs masked in-kernel
     if (n >= 98304) return 20; // super-tile pairs, 2 per lane, 2 per item
-    if (n >= 20480) return 19; // super-tile pairs, 2 per lane, 1 per item
-    if (n >= 1024) return 18;  // tile pairs, 2 per lane
+    if (n >= 32768) return 19; // super-tile pairs, 2 per lane, 1 per item
+    if (n >= 96) return 18;    // tile pairs, 2 per lane
   }
   if (n >= (size_t)1 << 17) return 8; // 256 x 1, split 2
   if (n < 4096) return 8;

@@ -174,45 +174,48 @@ int forward_default_config(size_t n, int mode) {
   // float at the cost of the diagonal passes only: same choice
   if (mode == MODE_PLAIN_SKIP) mode = MODE_PLAIN;
   if (mode == MODE_KAHAN_SKIP) mode = MODE_KAHAN;
-  // Measured on MI355X (disk ICs), us per step.  Tile pairs, 2 per lane
-  // (two items per tile pair below 6656: n = 4096 15.5, 6144 20.9; one item
-  // with priority steps from there: 7168 23.1, 8192 27.2; see
-  // launch_forward_sym): n = 4096 22.6 (target-sharded 128 x 1 split 8: 29), 8192 38.1 (38.7),
-  // 12800 57.5 (82.5), 32768 238.4 (323.6; 4 per lane 266.3).  Super-tile
-  // pairs, 2 per lane, 1 / 2 per item: 49152 481.8 / 532.7 (tile pairs
-  // 499.0), 65536 810.7 / 842.7 (867.9), 98304 1764 / 1780 (4 per lane
-  // 1860, 8 per lane 1915), 131072 3118 / 3104 (4 per lane 3176, 8 per lane
-  // 3299), 262144 12236 / 12133 (8 per lane 11804).  Past 2^19 two
-  // super-tiles of 8 per lane per item run as fast as one and need 25 %
-  // less scratch (6042 Gint/s at 2^20); past 2^20 four per item keep the
-  // partials at 16 GB for 2^21 particles, and past 2^21 the step runs in
-  // bands of source super-tiles with at most 8 GB of partials each (the
-  // 4-per-lane shape with 4 per item is banded past 2^20).
+  // Measured on MI355X (disk ICs), us per step (device time), best others in
+  // brackets.  Tile pairs, 2 per lane: n = 4097 13.5 (target-sharded 40), 12000
+  // 38.2 (super-tiles of 512, 1 per item 49.8), 28000 141.1 (150.5), 32768
+  // 189.4 (191.6), 36000 227.6 (222.0), 49000 405.5 (387.5).  Super-tiles win
+  // from about 34000; the line stays at 49152 because the tile pairs' partials
+  // (64 to 217 MiB at 26752 to 49151) are what makes the allocation-free step
+  // refuse those sizes, and super-tiles (54 MiB) would have it accept them.
+  // Super-tiles of 512, 1 per item: 50021 379 (tile pairs 412, 1024 412), 52000
+  // 426.2 (453.8), 65536 652 (677 with 1024), 100000 1465 (1468 with 2 per
+  // item, 1470 with 1024).  Of 1024:
+  // 131072 2489 (2496 with 512, 2605 with 2048), 200000 5734 (5757, 5789),
+  // 262144 9786 (2048: 9868, with a quarter of the scratch's growth: the
+  // choice from there).  Past 2^19 two super-tiles of 2048 per item need 25 %
+  // less scratch; past 2^20 four per item keep the partials at 16 GB for 2^21
+  // particles, and past 2^21 the step runs in bands of source super-tiles with
+  // at most 8 GB of partials each (the 4-per-lane shape with 4 per item is
+  // banded past 2^20).
   if (mode == MODE_PLAIN && n <= kSymBandedMaxParticles) {
     if (n > kSymMaxParticles) return 24; // 8 per lane, 4 per item (banded past 2^21)
-    if (n > ((size_t)1 << 19)) return 23; // symmetric, 8 per lane, 2 per item
+    if (n > ((size_t)1 << 19)) return 23;  // symmetric, 8 per lane, 2 per item
     if (n >= ((size_t)1 << 18)) return 22; // symmetric, 8 per lane, 1 per item
-    if (n >= 98304) return 35;             // symmetric, 2 per lane, 2 per item
+    if (n >= ((size_t)1 << 17)) return 25; // symmetric, 4 per lane, 1 per item
     if (n >= 49152) return 34;             // symmetric, 2 per lane, 1 per item
     if (n >= 6656) return 33;              // symmetric tile pairs, 2 per lane
     if (n >= 4096) return 37;              // the same, two items per tile pair
   }
-  // Kahan, Gint/s: tile pairs, 2 per lane: n = 16384 1961 (best
-  // target-sharded 1664), 32768 2408 (1847); super-tile pairs, 2 per lane,
-  // 1 / 2 per item: 65536 2774 / 2674, 131072 2873 / 2867, 262144 2916 /
-  // 2929 (4 per lane 2411, target-sharded 2373).  The compensated sums'
-  // dependency chains bound this mode, so the shapes with the most waves
-  // win; below 12288 the target-sharded ones (8192: 1229 vs 1128).  Above
-  // 2^18 four super-tiles per item run in bands of source super-tiles (16 GB
-  // of (sum, compensation) partials per band).
+  // Kahan, us per step: tile pairs, 2 per lane: n = 300 9.9 (best
+  // target-sharded 24), 4097 20 (56), 12000 67 (123), 32000 324 (572);
+  // super-tiles of 512, 1 per item, and tile pairs: 32768 362.6 and 353.8,
+  // 36000 421.9 and 427.0, 40960 517.8 and 540.3, 49000 738.2 and 765.4 (below
+  // 40960 the same reason as above).  1 / 2 per item: 100000 2830 / 2809,
+  // 262144 19295 / 18999 (target-sharded 28751).  Above 2^18 four super-tiles
+  // per item run in bands of source super-tiles (16 GB of (sum, compensation)
+  // partials per band).
   if (mode == MODE_KAHAN) {
     if (n > ((size_t)1 << 18) && n <= kSymBandedMaxParticles)
       return 36;               // symmetric, 2 per lane, 4 per item, banded
     if (n >= ((size_t)1 << 17) && n <= ((size_t)1 << 18))
       return 35;               // symmetric, 2 per lane, 2 per item
-    if (n >= 49152 && n < ((size_t)1 << 17))
+    if (n >= 40960 && n < ((size_t)1 << 17))
       return 34;               // symmetric, 2 per lane, 1 per item
-    if (n >= 12288 && n < 49152)
+    if (n >= 64 && n < 40960)
       return 33;               // symmetric tile pairs, 2 per lane
   }
   // Target-sharded, Gint/s: n = 4096: 128 x 1 split 8 629 (256 x 1 split 8

@@ -461,16 +461,17 @@ __device__ __forceinline__ bool combine_runs(float (&f)[R::ACC],
 // sets of 64 sources, one source per lane and step.  Per step a lane reads
 // one source (SRC floats) from LDS and rotates ACC reaction sums for U pair
 // terms; no barrier inside a row.
-//   * U = 8 or 4: wave w meets sets w, w + 4, .. of GB;  U = 2: two waves
-//     share a set, each half of its 64 steps, and add their reaction sums
+//   * U = 8 or 4: wave w meets sets w, w + W, .. of GB;  U = 2: W / 2 waves
+//     share a set, each its part of the 64 steps, and add their reaction sums
 //     through LDS;
 //   * at the end of a row the waves' target sums are added in a fixed tree,
 //     (0 + 2) + (1 + 3);
 //   * M = 1: the row meets every GB of the work item before that;  M > 1: the
 //     rows of GA meet one GB in turn, and the reaction sums of a set, owned by
 //     one wave, wait in LDS from row to row (one reaction partial per ST x ST
-//     pairs, 1 / M of M = 1's).  M = 4 runs 8 waves per workgroup: half as
-//     long items, a shorter last round for the same partials.
+//     pairs, 1 / M of M = 1's).  M = 4 runs W = 8 waves per workgroup, the
+//     others 4: half as long items, a shorter last round for the same
+//     partials.
 // The sources lie twice in LDS (128 floats per coordinate and wave), so that
 // step s reads at lane + s with no wrap, its offset in the instruction.
 //
@@ -481,15 +482,17 @@ __device__ __forceinline__ bool combine_runs(float (&f)[R::ACC],
 // 2 x 2 -> 8 x 1: forward 56 -> 47, adjoint 85 -> 72, fused 120 -> 94, Kahan
 // 102 -> 89.  8 x 8 in four-wave passes with a barrier per pass: 50 (3 waves
 // per SIMD, 48 KiB of LDS).
-template <class R, int U, int M = 1>
+// W: waves per workgroup.  8 with M = 4; with U = 2, 8 where one wave per
+// SIMD would be all there is (see kTileWide).
+template <class R, int U, int M, int W_ = (M > 2 ? 8 : 4)>
 struct RowShape {
   static_assert(U == 2 || U == 4 || U == 8, "targets per lane");
   static_assert(M == 1 || U == 8, "rows per super-tile");
   static constexpr int RT = 64 * U;                  // row
   static constexpr int ST = RT * M;                  // super-tile
-  static constexpr int W = M > 2 ? 8 : 4;            // waves per workgroup
+  static constexpr int W = W_;
   static constexpr int SETS = ST / 64;               // source sets
-  static constexpr int PARTS = U >= 4 ? 1 : 4 / U;   // waves per set
+  static constexpr int PARTS = U >= 4 ? 1 : W / SETS; // waves per set
   static constexpr int STEPS = 64 / PARTS;           // steps of a wave per set
   // LDS: the waves' sources, and in the same place (a barrier between) the
   // two buffers of the tree; then the reaction sums that wait or meet there
@@ -520,12 +523,11 @@ __device__ __forceinline__ void wave_lds_fence() {
 // mod 64 into rs.  masked: sources at or past index `valid` of the set and,
 // in the set of the wave's own targets self (-1: another set), the self pairs
 // (step 0) contribute nothing.
-template <class R, int U>
+template <class R, int U, int STEPS>
 __device__ __forceinline__ void
 row_pass(const float (&t)[U][R::SRC], float (&a)[U][R::ACC],
          float (&rs)[R::ACC], const float *src, int lane, int s0, float eps,
          bool masked, int self, int valid) {
-  constexpr int STEPS = RowShape<R, U>::STEPS;
   const float *p = src + lane + s0;
   if (!masked) {
 #pragma unroll 4
@@ -561,12 +563,11 @@ row_pass(const float (&t)[U][R::SRC], float (&a)[U][R::ACC],
 // On the diagonal (gb == ga) a row meets its own sets without reactions (each
 // of their pairs twice) and, M > 1, those of the rows after it with; their
 // reaction sums wait for those rows in LDS (add_waves subtracts them).
-template <class R, int U, int M, class SpAt>
+template <class R, class S, int U, int M, class SpAt>
 __device__ __forceinline__ void meet_sources(float (&sum)[U][R::ACC],
                                              const SymArgs &a, float *lds,
                                              int ga, int row, int gb0, int gb1,
                                              SpAt sp_at) {
-  using S = RowShape<R, U, M>;
   constexpr int ST = S::ST;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int part = w % S::PARTS, first = w / S::PARTS;
@@ -612,8 +613,8 @@ __device__ __forceinline__ void meet_sources(float (&sum)[U][R::ACC],
     // not kept)
     if (M > 1 && row > 0) R::fetch(rs, held, ST);
     if (left > 0) // the same for the waves that share a set
-      row_pass<R, U>(t, sum, rs, src, lane, s0, a.c.eps, masked,
-                     g == ga ? set - row * U : -1, left);
+      row_pass<R, U, S::STEPS>(t, sum, rs, src, lane, s0, a.c.eps, masked,
+                               g == ga ? set - row * U : -1, left);
     if (g == ga && (M == 1 || set < (row + 1) * U)) continue;
     if constexpr (S::PARTS == 1) {
       const bool out = M == 1 || (row == M - 1 && g > ga);
@@ -715,14 +716,13 @@ __device__ __forceinline__ void add_waves(float (&sum)[U][R::ACC], float *lds,
 
 // Work item: super-tile ga against source super-tiles [gb0, gb1), gb0 >= ga.
 // Row partial ([ACC][ST]) to fp, reaction sums to sp_at(gb) ([ACC][ST]).
-template <class R, int U, int M, class SpAt>
+template <class R, class S, int U, int M, class SpAt>
 __device__ __forceinline__ void row_item(const SymArgs &a, float *lds, int ga,
                                          int gb0, int gb1, float *fp,
                                          SpAt sp_at) {
-  using S = RowShape<R, U, M>;
   float sum[U][R::ACC];
   if constexpr (M == 1) {
-    meet_sources<R, U, M>(sum, a, lds, ga, 0, gb0, gb1, sp_at);
+    meet_sources<R, S, U, M>(sum, a, lds, ga, 0, gb0, gb1, sp_at);
     add_waves<R, U, S::W, false>(sum, lds, nullptr, fp, S::ST);
   } else {
 #pragma unroll 1
@@ -731,7 +731,7 @@ __device__ __forceinline__ void row_item(const SymArgs &a, float *lds, int ga,
       for (int row = 0; row < M; ++row) {
         // rows of padding only: the last super-tile's, which has no reactions
         if (ga * S::ST + row * S::RT >= a.n) break;
-        meet_sources<R, U, M>(sum, a, lds, ga, row, gb, gb + 1, sp_at);
+        meet_sources<R, S, U, M>(sum, a, lds, ga, row, gb, gb + 1, sp_at);
         const float *held =
             gb == ga && row > 0 ? lds + S::REACT + row * S::RT : nullptr;
         float *f = fp + row * S::RT;
@@ -773,15 +773,16 @@ __device__ __forceinline__ void sym_item(long long it, int ts, int L, int &ga,
   }
 }
 
-template <class R, int U, int M>
-__global__ __launch_bounds__((64 * RowShape<R, U, M>::W)) void sym_kernel(SymArgs a) {
-  __shared__ float lds[RowShape<R, U, M>::LDS_FLOATS];
-  constexpr int ST = RowShape<R, U, M>::ST;
+template <class R, int U, int M, int W>
+__global__ __launch_bounds__(64 * W) void sym_kernel(SymArgs a) {
+  using S = RowShape<R, U, M, W>;
+  constexpr int ST = S::ST;
+  __shared__ float lds[S::LDS_FLOATS];
   const int ts = a.ts, L = a.chunk;
   int ga, c;
   sym_item(blockIdx.x, ts, L, ga, c);
   const int gb0 = ga + c * L;
-  row_item<R, U, M>(
+  row_item<R, S, U, M>(
       a, lds, ga, gb0, min(gb0 + L, ts),
       a.fpart + (size_t)(row_first(ga, ts, L) + c) * (R::ACC * ST),
       [&](int gb) {
@@ -862,18 +863,19 @@ __device__ __forceinline__ void band_item(long long it, int b0, int W, int L,
   }
 }
 
-template <class R, int U, int M>
-__global__ __launch_bounds__((64 * RowShape<R, U, M>::W)) void sym_band_kernel(SymArgs a) {
-  __shared__ float lds[RowShape<R, U, M>::LDS_FLOATS];
-  constexpr int ST = RowShape<R, U, M>::ST;
-  const int L = a.chunk, b0 = a.b0, W = a.bw;
+template <class R, int U, int M, int W>
+__global__ __launch_bounds__(64 * W) void sym_band_kernel(SymArgs a) {
+  using S = RowShape<R, U, M, W>;
+  constexpr int ST = S::ST;
+  __shared__ float lds[S::LDS_FLOATS];
+  const int L = a.chunk, b0 = a.b0, bw = a.bw;
   const long long it = blockIdx.x;
   int ga, gb0;
-  band_item(it, b0, W, L, ga, gb0);
-  row_item<R, U, M>(
-      a, lds, ga, gb0, min(gb0 + L, b0 + W),
+  band_item(it, b0, bw, L, ga, gb0);
+  row_item<R, S, U, M>(
+      a, lds, ga, gb0, min(gb0 + L, b0 + bw),
       a.fpart + (size_t)it * (R::ACC * ST), [&](int gb) {
-        return a.spart + (size_t)band_pair_slot(ga, gb, b0, W) * (R::ACC * ST);
+        return a.spart + (size_t)band_pair_slot(ga, gb, b0, bw) * (R::ACC * ST);
       });
 }
 
@@ -1002,12 +1004,12 @@ __device__ __forceinline__ void leave_queue(const SymBatchArgs &b) {
   }
 }
 
-template <int U, int M>
-__global__
-__launch_bounds__((64 * RowShape<ForceRule, U, M>::W), 4) void sym_batch_kernel(SymBatchArgs b) {
+template <int U, int M, int W>
+__global__ __launch_bounds__(64 * W, 4) void sym_batch_kernel(SymBatchArgs b) {
   using R = ForceRule;
-  constexpr int ST = RowShape<R, U, M>::ST;
-  __shared__ float lds[RowShape<R, U, M>::LDS_FLOATS];
+  using S = RowShape<R, U, M, W>;
+  constexpr int ST = S::ST;
+  __shared__ float lds[S::LDS_FLOATS];
   __shared__ int s_item;
   for (;;) {
     const int item = next_item(b, &s_item);
@@ -1015,7 +1017,7 @@ __launch_bounds__((64 * RowShape<ForceRule, U, M>::W), 4) void sym_batch_kernel(
     const int4 it = b.items[item];
     const SymArgs a = system_view(b, it.x, ST);
     float *slot = b.part + (size_t)it.w * (2 * R::ACC * ST);
-    row_item<R, U, M>(a, lds, it.y, it.z, it.z + 1, slot,
+    row_item<R, S, U, M>(a, lds, it.y, it.z, it.z + 1, slot,
                       [&](int) { return slot + R::ACC * ST; });
   }
   leave_queue(b);
@@ -1061,32 +1063,45 @@ struct SymShape {
   KernelFn pairs, finalize;
 };
 
-template <class R, int U, int M, int RUNS>
+template <class R, int U, int M, int RUNS, int W = (M > 2 ? 8 : 4)>
 constexpr SymShape sym_shape() {
   constexpr int ST = 64 * U * M;
-  return {ST, 64 * RowShape<R, U, M>::W, RUNS, sym_kernel<R, U, M>,
-          sym_finalize<R, ST, RUNS>};
+  return {ST, 64 * W, RUNS, sym_kernel<R, U, M, W>, sym_finalize<R, ST, RUNS>};
 }
 
 // Targets per lane of a tile-pair shape: `unroll` particles per lane and
-// tile (tiles of 64 * unroll), `items` work items per tile pair.  Tiles of 2
-// per lane are taken two at a time (4 targets per lane), one at a time with
-// two items per tile pair.
-int tile_targets(int unroll, int items) {
-  return unroll == 2 && items == 1 ? 4 : unroll;
+// tile (tiles of 64 * unroll), `items` work items per tile pair.  With two
+// items, and below kTilePairRows particles, tiles of 2 per lane are taken one
+// at a time (super-tiles of 128, two waves per set of sources: four times the
+// workgroups); from there two at a time (4 targets per lane, half the LDS
+// traffic and partials per pair term).  Both sides, us per step, device time
+// (forward / Kahan / adjoint / fused): n = 4097 13.4 / 20 / 17 / 21 vs 19.4 /
+// 28 / 24 / 31, 9000 27.5 / 46.7 / 38.6 / 50.9 vs 27.2 / 47.3 / 41.1 / 52.7,
+// 12000 42.1 / 71.3 / 59.1 / 78.9 vs 38.2 / 67.2 / 57.0 / 75.9.
+// Below kTileWide particles 8 waves share the 128 x 128 pairs, each a quarter
+// of a set's steps: with fewer pairs than SIMDs the step is the latency of
+// one wave (n = 1000 8.9 / 11.0 / 10.0 / 11.9 vs 10.2 / 12.9 / 12.0 / 14.1,
+// 4097 13.8 / 20.7 / 17.4 / 21.5 vs 13.4 / 20.0 / 17.1 / 21.3).
+constexpr size_t kTilePairRows = 9728;
+constexpr size_t kTileWide = 3328;
+
+int tile_targets(int unroll, int items, size_t n) {
+  return unroll == 2 && items == 1 && n >= kTilePairRows ? 4 : unroll;
 }
 
 // Super-tile shapes: M = unroll / 2 rows of 512.  Tile pairs: one row per
 // super-tile, of one tile or a pair of tiles.
 template <class R>
-const SymShape *find_shape(int unroll, bool tiles, int items) {
-  static const SymShape tile2 = sym_shape<R, 2, 1, kTileRuns>(),
+const SymShape *find_shape(int unroll, bool tiles, int items, size_t n) {
+  static const SymShape wide2 = sym_shape<R, 2, 1, kTileRuns, 8>(),
+                        tile2 = sym_shape<R, 2, 1, kTileRuns>(),
                         tile4 = sym_shape<R, 4, 1, kTileRuns>(),
                         rows1 = sym_shape<R, 8, 1, 1>(),
                         rows2 = sym_shape<R, 8, 2, 1>();
   if (tiles) {
     if (unroll != 2 && unroll != 4) return nullptr;
-    return tile_targets(unroll, items) == 2 ? &tile2 : &tile4;
+    if (tile_targets(unroll, items, n) == 4) return &tile4;
+    return n < kTileWide ? &wide2 : &tile2;
   }
   if (unroll == 2) return &rows1;
   if (unroll == 4) return &rows2;
@@ -1113,7 +1128,8 @@ struct BandShape {
 // Band kernels of rule R: 2, 4 or 8 particles per lane (Kahan: 2 or 4).
 template <class R, int M>
 constexpr BandShape band_shape() {
-  return {2 * M, 512 * M, 64 * RowShape<R, 8, M>::W, sym_band_kernel<R, 8, M>,
+  constexpr int W = RowShape<R, 8, M>::W;
+  return {2 * M, 512 * M, 64 * W, sym_band_kernel<R, 8, M, W>,
           sym_band_fold<R, 512 * M>, sym_band_finish<R>};
 }
 
@@ -1252,7 +1268,7 @@ size_t sym_scratch_bytes(int unroll, int chunk, size_t n, int acc,
     // second tile on
     const long long P = 64LL * unroll;
     const long long T = ((long long)n + P - 1) / P;
-    const long long st = 64LL * tile_targets(unroll, chunk);
+    const long long st = 64LL * tile_targets(unroll, chunk, n);
     const long long ts = ((long long)n + st - 1) / st;
     return sizeof(float) * acc *
            (size_t)std::max(T * (T + 1) * P * std::max(chunk, 1), ts * ts * st);
@@ -1304,7 +1320,8 @@ int sym_batch_layout(int unroll, const int *sys_off, int num_systems,
 
 namespace {
 template <int U> const void *batch_pairs_fn() {
-  return reinterpret_cast<const void *>(sym_batch_kernel<8, U / 2>);
+  return reinterpret_cast<const void *>(
+      sym_batch_kernel<8, U / 2, RowShape<ForceRule, 8, U / 2>::W>);
 }
 template <int U> const void *batch_finalize_fn() {
   return reinterpret_cast<const void *>(sym_batch_finalize<256 * U>);
@@ -1386,10 +1403,10 @@ int launch_forward_sym(const StepConsts &c, int unroll, int chunk, bool tiles,
                      "two items per tile pair: plain sums, 2 per lane only");
   if (kahan)
     return launch_sym(
-        find_shape<KahanForceRule>(unroll, tiles, chunk), a, unroll, chunk, n,
+        find_shape<KahanForceRule>(unroll, tiles, chunk, (size_t)n), a, unroll, chunk, n,
         scratch, KahanForceRule::ACC, tiles, stream,
         tiles ? nullptr : find_band_shape<KahanForceRule>(unroll));
-  return launch_sym(find_shape<ForceRule>(unroll, tiles, chunk), a, unroll,
+  return launch_sym(find_shape<ForceRule>(unroll, tiles, chunk, (size_t)n), a, unroll,
                     chunk, n, scratch, ForceRule::ACC, tiles, stream,
                     tiles ? nullptr : find_band_shape<ForceRule>(unroll));
 }
@@ -1420,11 +1437,11 @@ int launch_adjoint_sym(const StepConsts &c, bool fused, int unroll, int chunk,
     a.ny = nxt[1];
     a.nz = nxt[2];
     return launch_sym(
-        find_shape<AdjointRule<true>>(unroll, tiles, chunk), a, unroll, chunk, n,
+        find_shape<AdjointRule<true>>(unroll, tiles, chunk, (size_t)n), a, unroll, chunk, n,
         scratch, AdjointRule<true>::ACC, tiles, stream,
         tiles ? nullptr : find_band_shape<AdjointRule<true>>(unroll));
   }
-  return launch_sym(find_shape<AdjointRule<false>>(unroll, tiles, chunk), a, unroll,
+  return launch_sym(find_shape<AdjointRule<false>>(unroll, tiles, chunk, (size_t)n), a, unroll,
                     chunk, n, scratch, AdjointRule<false>::ACC, tiles, stream,
                     tiles ? nullptr : find_band_shape<AdjointRule<false>>(unroll));
 }
