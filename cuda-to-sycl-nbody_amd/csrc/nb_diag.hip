@@ -29,7 +29,8 @@
 // particles the potential is off by 0.55 u in the mean and 1.73 u at most
 // (before 0.63 and 1.83); forces over 500 targets by 0.9 to 1.4e-16 in the
 // mean (before 3.2 to 7.6e-16).
- <algorithm>
+
+#include <algorithm>
 #include <type_traits>
 #include <vector>
 
