@@ -95,6 +95,139 @@ __global__ __launch_bounds__(256) void fwd_finalize(FwdArgs a) {
                 a.nx, a.ny, a.nz);
 }
 
+// ---- one launch for small systems -----------------------------------------
+//
+// Below a few thousand particles a step is latency: two launches, a source
+// loop with few waves, a second trip through memory for the partial sums.
+// Here a workgroup of 16 waves owns 4 * U targets and all their sources: each
+// row of 16 lanes holds U targets, the 16 waves x 16 lanes stride through the
+// sources in batches of four loads (the next batch is in flight during the
+// pairs), four DPP adds sum a row, LDS brings the 16 waves' sums together, and
+// the lanes that integrate have loaded their particles at the start.
+// Device time at n = 1000 3.4 us, 4000 8.9 (split shapes and a second kernel:
+// 23.8, 24.8); the launch and two dependent trips to L2 are about 3 of it.
+
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallLanes = 16;                         // source lanes per row
+constexpr int kSmallStride = kSmallBlock / 64 * kSmallLanes; // sources per pass
+constexpr int kSmallBatch = 4;
+
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
+                                         0xf, 0xf, false));
+}
+
+// (s, c) stands for s - c.  TwoSum keeps the rounding of s + s' in c.
+__device__ __forceinline__ void meet(float &s, float &c, float s2, float c2) {
+  const float t = s + s2;
+  const float b = t - s;
+  const float err = (s - (t - b)) + (s2 - b);
+  c = (c + c2) - err;
+  s = t;
+}
+
+template <bool KAHAN, int CTRL>
+__device__ __forceinline__ void row_step(float &s, float &c) {
+  if constexpr (KAHAN)
+    meet(s, c, dpp<CTRL>(s), dpp<CTRL>(c));
+  else
+    s = s + dpp<CTRL>(s);
+}
+
+// Sum over a row of 16 lanes, in every lane of it (row_ror 8, 4, 2, 1).
+template <bool KAHAN>
+__device__ __forceinline__ void row_sum(float &s, float &c) {
+  row_step<KAHAN, 0x128>(s, c);
+  row_step<KAHAN, 0x124>(s, c);
+  row_step<KAHAN, 0x122>(s, c);
+  row_step<KAHAN, 0x121>(s, c);
+}
+
+template <int U, int MODE>
+__global__ __launch_bounds__(kSmallBlock) void fwd_small_kernel(FwdArgs a) {
+  constexpr bool KAHAN = MODE == MODE_KAHAN || MODE == MODE_KAHAN_SKIP;
+  constexpr int NT = 4 * U;                  // targets per workgroup
+  constexpr int WAVES = kSmallBlock / 64;
+  constexpr int NV = KAHAN ? 6 : 3;
+  static_assert(WAVES == kSmallLanes, "one lane of a row per wave's sum");
+  __shared__ float sums[NV][NT][WAVES];
+  const int n = a.n;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = lane >> 4, sl = lane & 15;
+  const int first = blockIdx.x * NT;
+
+  // lane 0 of row r (of the workgroup) integrates target first + r
+  const int fin = threadIdx.x >> 4;
+  const bool owner = sl == 0 && fin < NT && first + fin < n;
+  Particle own = {};
+  if (owner)
+    own = load_particle(first + fin, a.px, a.py, a.pz, a.vx, a.vy, a.vz);
+
+  Targets<U, MODE> T;
+  T.load(a.px, a.py, a.pz, first + row * U, 1, 0, n);
+
+  const int s0 = wave * kSmallLanes + sl;
+  constexpr int B = kSmallBatch, PASS = kSmallStride * B;
+  float X[B], Y[B], Z[B];
+  auto fetch = [&](int b) {
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      const int j = min(b + q * kSmallStride + s0, n - 1);
+      X[q] = a.px[j];
+      Y[q] = a.py[j];
+      Z[q] = a.pz[j];
+    }
+  };
+  fetch(0);
+  for (int b = 0; b < n; b += PASS) {
+    float x[B], y[B], z[B];
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      x[q] = X[q];
+      y[q] = Y[q];
+      z[q] = Z[q];
+    }
+    if (b + PASS < n) fetch(b + PASS);
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      const int j = b + q * kSmallStride + s0;
+      if (j < n) T.one(x[q], y[q], z[q], j, a.c.eps);
+    }
+  }
+
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    row_sum<KAHAN>(T.ax[k], T.cx[k]);
+    row_sum<KAHAN>(T.ay[k], T.cy[k]);
+    row_sum<KAHAN>(T.az[k], T.cz[k]);
+    if (sl == 0) {
+      sums[0][row * U + k][wave] = T.ax[k];
+      sums[1][row * U + k][wave] = T.ay[k];
+      sums[2][row * U + k][wave] = T.az[k];
+      if constexpr (KAHAN) {
+        sums[3][row * U + k][wave] = T.cx[k];
+        sums[4][row * U + k][wave] = T.cy[k];
+        sums[5][row * U + k][wave] = T.cz[k];
+      }
+    }
+  }
+  __syncthreads();
+  if (wave >= U) return; // NT rows of 16 lanes are U waves
+  float f[3], c[3] = {};
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    f[m] = sums[m][fin][sl];
+    if constexpr (KAHAN) c[m] = sums[3 + m][fin][sl];
+    row_sum<KAHAN>(f[m], c[m]);
+    if constexpr (KAHAN) f[m] = f[m] - c[m];
+  }
+  if (owner)
+    integrate_loaded(a.c, first + fin, own, f[0], f[1], f[2], a.vx, a.vy, a.vz,
+                     a.nx, a.ny, a.nz);
+}
+
 using KernelFn = void (*)(FwdArgs);
 
 template <int BLOCK, int U, int TILE>
@@ -113,6 +246,18 @@ KernelFn shape_kernel(int mode, bool split) {
     return nullptr;
   }
 #undef NB_MODE_CASE
+}
+
+template <int U>
+KernelFn small_kernel(int mode) {
+  switch (mode) {
+  case MODE_PLAIN: return fwd_small_kernel<U, MODE_PLAIN>;
+  case MODE_PLAIN_SKIP: return fwd_small_kernel<U, MODE_PLAIN_SKIP>;
+  case MODE_KAHAN: return fwd_small_kernel<U, MODE_KAHAN>;
+  case MODE_KAHAN_SKIP: return fwd_small_kernel<U, MODE_KAHAN_SKIP>;
+  case MODE_PREDICATED: return fwd_small_kernel<U, MODE_PREDICATED>;
+  default: return nullptr;
+  }
 }
 
 struct ShapeEntry {
@@ -153,6 +298,7 @@ const FwdConfig kConfigs[] = {
     {256, 2, 512, 1, SCHEME_SYMMETRIC}, {256, 2, 512, 2, SCHEME_SYMMETRIC},
     {256, 2, 512, 4, SCHEME_SYMMETRIC},
     {256, 2, 128, 2, SCHEME_SYMMETRIC_TILES}, // two items per tile pair
+    {kSmallBlock, 1, 1024, 1},                // one launch (fwd_small_kernel)
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 
@@ -162,6 +308,12 @@ KernelFn find_kernel(const FwdConfig &c, int mode) {
       return s.get(mode, c.split > 1);
   return nullptr;
 }
+
+// Targets per row of the one-launch shape: as few as leave one workgroup for
+// each of the 256 CUs.  1 / 2 / 4 targets, us: n = 1000 3.4 / 3.6 / 4.3, 1500
+// 4.7 / 4.3 / 5.4, 2000 5.1 / 4.6 / 5.8, 3000 8.1 / 7.7 / 7.5, 4000 11.7 / 9.2
+// / 8.9.
+int small_targets(int n) { return n <= 1024 ? 1 : n <= 2048 ? 2 : 4; }
 
 } // namespace
 
@@ -200,8 +352,8 @@ int forward_default_config(size_t n, int mode) {
     if (n >= 6656) return 33;              // symmetric tile pairs, 2 per lane
     if (n >= 4096) return 37;              // the same, two items per tile pair
   }
-  // Kahan, us per step: tile pairs, 2 per lane: n = 300 9.9 (best
-  // target-sharded 24), 4097 20 (56), 12000 67 (123), 32000 324 (572);
+  // Kahan, us per step: tile pairs, 2 per lane: n = 4097 20 (best split
+  // target-sharded 56), 5000 22.2 (one launch 22.6), 12000 67 (123), 32000 324 (572);
   // super-tiles of 512, 1 per item, and tile pairs: 32768 362.6 and 353.8,
   // 36000 421.9 and 427.0, 40960 517.8 and 540.3, 49000 738.2 and 765.4 (below
   // 40960 the same reason as above).  1 / 2 per item: 100000 2830 / 2809,
@@ -215,9 +367,14 @@ int forward_default_config(size_t n, int mode) {
       return 35;               // symmetric, 2 per lane, 2 per item
     if (n >= 40960 && n < ((size_t)1 << 17))
       return 34;               // symmetric, 2 per lane, 1 per item
-    if (n >= 64 && n < 40960)
+    if (n >= 4096 && n < 40960)
       return 33;               // symmetric tile pairs, 2 per lane
   }
+  // One launch, plain / Kahan us (device time; split target-sharded plain,
+  // then tile pairs plain / Kahan): n = 64 2.9 / 3.5 (10.5, 6.4 / 8.0), 1000
+  // 3.4 / 4.2 (23.8, 8.5 / 10.6), 2000 4.6 / 6.7 (24.0, 9.0 / 11.2), 4000
+  // 8.9 / 15.3 (24.8, 11.9 / 17.6); tile pairs from 4096.
+  if (n < 4096) return 38;
   // Target-sharded, Gint/s: n = 4096: 128 x 1 split 8 629 (256 x 1 split 8
   // 480); 8192: 256 x 1 split 8 1746 (split 16 1629); 16384 .. 32768:
   // 256 x 1 split 16 2843 .. 3432 (split 8 2792 .. 3292); 65536: 256 x 4
@@ -263,7 +420,12 @@ int launch_forward(const StepConsts &c, int mode, int cfg, const float *px,
                               py, pz, vx, vy, vz, nx, ny, nz, n, scratch,
                               stream);
   }
-  KernelFn fn = find_kernel(fc, mode);
+  const bool small = fc.block == kSmallBlock;
+  const int per_row = small ? small_targets(n) : 0;
+  KernelFn fn = !small         ? find_kernel(fc, mode)
+                : per_row == 1 ? small_kernel<1>(mode)
+                : per_row == 2 ? small_kernel<2>(mode)
+                               : small_kernel<4>(mode);
   if (!fn) return set_error(NB_ERR_UNSUPPORTED, "no kernel for this mode");
   if (fc.split > 1 && !scratch)
     return set_error(NB_ERR_INVALID_ARG, "split launch needs scratch");
@@ -285,7 +447,7 @@ int launch_forward(const StepConsts &c, int mode, int cfg, const float *px,
   a.jchunk = ((per_chunk + fc.tile - 1) / fc.tile) * fc.tile;
   a.c = c;
 
-  const int targets = fc.block * fc.unroll;
+  const int targets = small ? 4 * per_row : fc.block * fc.unroll;
   dim3 grid((n + targets - 1) / targets, fc.split);
   dim3 block(fc.block);
   void *args[] = {&a};

@@ -27,24 +27,47 @@ namespace nb {
 
 // Integrator of src/simulator.cu:214-228 in source order (no contraction):
 //   v = v * damping;  v += (F * dt) * G;  x_next = x + v * dt
-__device__ __forceinline__ void integrate_ref(const StepConsts &c, int i,
-                                              float fx, float fy, float fz,
-                                              const float *px, const float *py,
-                                              const float *pz, float *vx,
-                                              float *vy, float *vz, float *nx,
-                                              float *ny, float *nz) {
-  float ux = vx[i] * c.damping;
-  float uy = vy[i] * c.damping;
-  float uz = vz[i] * c.damping;
+struct Particle {
+  float x, y, z, vx, vy, vz;
+};
+
+__device__ __forceinline__ Particle load_particle(int i, const float *px,
+                                                  const float *py,
+                                                  const float *pz,
+                                                  const float *vx,
+                                                  const float *vy,
+                                                  const float *vz) {
+  return {px[i], py[i], pz[i], vx[i], vy[i], vz[i]};
+}
+
+__device__ __forceinline__ void integrate_loaded(const StepConsts &c, int i,
+                                                 const Particle &p, float fx,
+                                                 float fy, float fz, float *vx,
+                                                 float *vy, float *vz,
+                                                 float *nx, float *ny,
+                                                 float *nz) {
+  float ux = p.vx * c.damping;
+  float uy = p.vy * c.damping;
+  float uz = p.vz * c.damping;
   ux = ux + (fx * c.dt) * c.G;
   uy = uy + (fy * c.dt) * c.G;
   uz = uz + (fz * c.dt) * c.G;
   vx[i] = ux;
   vy[i] = uy;
   vz[i] = uz;
-  nx[i] = px[i] + ux * c.dt;
-  ny[i] = py[i] + uy * c.dt;
-  nz[i] = pz[i] + uz * c.dt;
+  nx[i] = p.x + ux * c.dt;
+  ny[i] = p.y + uy * c.dt;
+  nz[i] = p.z + uz * c.dt;
+}
+
+__device__ __forceinline__ void integrate_ref(const StepConsts &c, int i,
+                                              float fx, float fy, float fz,
+                                              const float *px, const float *py,
+                                              const float *pz, float *vx,
+                                              float *vy, float *vz, float *nx,
+                                              float *ny, float *nz) {
+  integrate_loaded(c, i, load_particle(i, px, py, pz, vx, vy, vz), fx, fy, fz,
+                   vx, vy, vz, nx, ny, nz);
 }
 
 // Kahan step: s += r * inv with running compensation c (the product is
