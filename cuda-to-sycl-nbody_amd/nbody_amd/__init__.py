@@ -18,6 +18,7 @@ from typing import Sequence
 
 import numpy as np
 
+from ._rows import row_length, row_ptrs, stream_ptr
 from .diag import energy_momentum, forces_f64
 from .batch import Batch, batch_config_count, batch_config_info, plummer_batch_sizes
 from .adjoint import (adjoint_config_count, adjoint_config_info, adjoint_default_config,
@@ -263,10 +264,9 @@ def forward_step(params: NbParams, pos, vel, nxt, n: int | None = None, cfg: int
     """One stream-ordered step on device tensors: reads pos, updates vel in
     place, writes nxt (3 tensors each).  stream: a torch.cuda.Stream or None
     (the current stream)."""
-    import torch
-
-    n = int(pos[0].numel()) if n is None else int(n)
-    ptrs = _dev_ptrs(pos, n, "pos") + _dev_ptrs(vel, n, "vel") + _dev_ptrs(nxt, n, "nxt")
-    s = stream if stream is not None else torch.cuda.current_stream()
-    check(load().nb_forward_step_dev(ctypes.byref(params), *ptrs, n, cfg, acc,
-                                     ctypes.c_void_p(s.cuda_stream)))
+    n = row_length(pos) if n is None else int(n)
+    p = row_ptrs(pos, n) or _dev_ptrs(pos, n, "pos")
+    v = row_ptrs(vel, n) or _dev_ptrs(vel, n, "vel")
+    x = row_ptrs(nxt, n) or _dev_ptrs(nxt, n, "nxt")
+    check(load().nb_forward_step_dev(ctypes.byref(params), *p, *v, *x, n, cfg, acc,
+                                     stream_ptr(stream)))

@@ -14,11 +14,15 @@ from __future__ import annotations
 import ctypes
 
 from ._lib import NB_ERR_INVALID_ARG, NbParams, NbVec3, check, load
+from ._rows import row_length, row_ptrs, stream_ptr
 
 
 def _vec3(t, n: int) -> NbVec3:
     """A (3, n) contiguous float32 CUDA tensor, or a sequence of 3 tensors,
     each row holding at least n values."""
+    ptrs = row_ptrs(t, n)
+    if ptrs is not None:
+        return NbVec3(*ptrs)
     if len(t) != 3:
         raise ValueError("expected 3 rows (x, y, z)")
     rows = [t[0], t[1], t[2]]
@@ -31,28 +35,25 @@ def _vec3(t, n: int) -> NbVec3:
 
 
 def _stream(stream):
-    import torch
-
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    return ctypes.c_void_p(stream_ptr(stream))
 
 
 def adjoint_step(params: NbParams, pos, lam_x_next, lam_v_next, lam_x, lam_v, cfg: int = -1,
                  stream=None) -> None:
     """Cotangents of (x_n, v_n) from those of (x_{n+1}, v_{n+1}) at positions pos."""
-    n = int(pos[0].numel())
+    n = row_length(pos)
     vs = [_vec3(t, n) for t in (pos, lam_x_next, lam_v_next, lam_x, lam_v)]
-    check(load().nb_adjoint_step_dev(ctypes.byref(params), *[ctypes.byref(v) for v in vs], n,
-                                     cfg, _stream(stream)))
+    check(load().nb_adjoint_step_dev(ctypes.byref(params), *vs, n, cfg,
+                                     stream_ptr(stream)))
 
 
 def fwd_adjoint_step(params: NbParams, pos, vel, pos_next, lam_x_next, lam_v_next, lam_x, lam_v,
                      cfg: int = -1, stream=None) -> None:
     """Forward step (vel in place, pos_next written) and adjoint step at pos, one launch."""
-    n = int(pos[0].numel())
+    n = row_length(pos)
     vs = [_vec3(t, n) for t in (pos, vel, pos_next, lam_x_next, lam_v_next, lam_x, lam_v)]
-    check(load().nb_fwd_adjoint_step_dev(ctypes.byref(params), *[ctypes.byref(v) for v in vs],
-                                         n, cfg, _stream(stream)))
+    check(load().nb_fwd_adjoint_step_dev(ctypes.byref(params), *vs, n, cfg,
+                                         stream_ptr(stream)))
 
 
 def adjoint_default_config(n: int, params: NbParams | None = None) -> int:
