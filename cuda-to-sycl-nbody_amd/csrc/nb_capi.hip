@@ -182,8 +182,9 @@ struct nb_sim {
   float *staging_dev = nullptr; // the same memory, device address
   hipEvent_t ev_stage = nullptr;
   bool staged = false;
-  // Frames of two or more steps replay a captured hipGraph, one per start
-  // buffer, valid for the (steps, shape, pair mode, scratch) they hold.
+  // Frames of more than kDirectLaunches launches replay a captured hipGraph,
+  // one per start buffer, valid for the (steps, shape, pair mode, scratch)
+  // they hold.
   bool use_graph = true;
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   int graph_iters = 0, graph_cfg = -1, graph_mode = -1;
@@ -390,12 +391,21 @@ int nb_sim_create(const nb_params *p, const float *px, const float *py,
   return NB_OK;
 }
 
+// Launches of a frame up to which they are issued one by one: a graph costs
+// some 16 us before its first kernel, direct launches fall behind from the
+// sixth on.  Frame, graph / direct, us: n = 500 2 steps 36.7 / 19.3, 5 38.0 /
+// 29.5, 6 40 / 51, 8 45 / 56 (one launch a step); 4097 2 steps 47.5 / 38.4, 3
+// 58.4 / 59, 8 120 / 123; 20000 2 steps 189 / 178 (two launches a step).
+static constexpr long long kDirectLaunches = 5;
+
 int nb_sim_advance(nb_sim *s, int iters) {
   if (!s) return set_error(NB_ERR_INVALID_ARG, "sim is NULL");
   if (iters < 0) return set_error(NB_ERR_INVALID_ARG, "iters < 0");
   if (s->n == 0) return NB_OK;
   const int mode = pair_mode(s->p.calc_method, s->acc, s->p.dist_eps);
-  if (!s->use_graph || iters < 2) return launch_steps(s, iters, mode);
+  if (!s->use_graph ||
+      (long long)iters * forward_launches(s->cfg) <= kDirectLaunches)
+    return launch_steps(s, iters, mode);
   if (s->graph_iters != iters || s->graph_cfg != s->cfg ||
       s->graph_mode != mode || s->graph_scratch != s->scratch) {
     int st = hip_check(hipStreamSynchronize(s->stream), "stream synchronize");

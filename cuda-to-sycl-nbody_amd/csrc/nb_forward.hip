@@ -385,6 +385,11 @@ int forward_default_config(size_t n, int mode) {
   return 30;                           // 128 x 1, tile 512, split 8
 }
 
+int forward_launches(int cfg) {
+  const FwdConfig &c = kConfigs[cfg];
+  return c.scheme == SCHEME_TARGETS && c.split == 1 ? 1 : 2;
+}
+
 size_t forward_scratch_bytes(int cfg, size_t n, int mode) {
   const FwdConfig &c = kConfigs[cfg];
   if (c.scheme != SCHEME_TARGETS) // (sum, compensation) pairs for Kahan

@@ -156,6 +156,8 @@ int launch_forward(const StepConsts &c, int mode, int cfg, const float *px,
                    float *scratch, hipStream_t stream);
 
 // Bytes of scratch launch_forward needs for (cfg, n, pair mode).
+// Kernel launches of one step (a banded step takes more).
+int forward_launches(int cfg);
 size_t forward_scratch_bytes(int cfg, size_t n, int mode);
 
 // Scratch owned by the library: one buffer per (device, stream), grown on

@@ -178,8 +178,8 @@ class Simulator:
         check(self._lib.nb_sim_set_config(self._h, cfg))
 
     def set_graph(self, enable: bool) -> None:
-        """Replay frames of two or more steps from a captured hipGraph (the
-        default) or launch every step directly."""
+        """Replay frames of more than five launches from a captured hipGraph
+        (the default) or launch every step directly."""
         check(self._lib.nb_sim_set_graph(self._h, int(bool(enable))))
 
     @property

@@ -162,7 +162,8 @@ int nb_sim_set_accumulation(nb_sim *s, int mode);
 /* Changes simIterationsPerFrame for later nb_sim_step calls. */
 int nb_sim_set_frame_iterations(nb_sim *s, int iters);
 
-/* Frames of two or more steps (nb_sim_step, nb_sim_advance) are captured once
+/* Frames of more than five launches (a step takes one launch below 4096
+ * particles, two from there; nb_sim_step, nb_sim_advance) are captured once
  * as a hipGraph per (steps, launch shape, accumulation, start buffer) and
  * replayed; enable = 0 launches every step directly (results are the same
  * bits).  No counterpart in the reference, whose stepSim launches each step
