@@ -76,13 +76,15 @@ __device__ __forceinline__ float lds_rol1(float v) {
 }
 
 // sum_{l=1..m} ceil(l / L): work items of the rows of lengths 1..m.
-__host__ __device__ inline long long items_upto(long long m, int L) {
-  const long long q = m / L, r = m % L;
-  return (long long)L * q * (q + 1) / 2 + r * (q + 1);
+__host__ __device__ inline long long items_upto(int m, int L) {
+  const int q = m / L, r = m - q * L; // (a 64-bit division is 150 instructions)
+  return (long long)L * q * (q + 1) / 2 + (long long)r * (q + 1);
 }
 
 // First work item (= row-partial slot) of row ga.
 __host__ __device__ inline long long row_first(int ga, int ts, int L) {
+  if (L == 1) // no 64-bit division in the shapes of one super-tile per item
+    return (long long)ga * ts - (long long)ga * (ga - 1) / 2;
   return items_upto(ts, L) - items_upto(ts - ga, L);
 }
 
@@ -184,10 +186,15 @@ struct ForceRule : PlainPartials<3> {
     rs[2] = __builtin_fmaf(rz, K, rs[2]);
   }
 
+  using Own = Particle;
+  static __device__ __forceinline__ Own own(const SymArgs &a, int i) {
+    return load_particle(i, a.px, a.py, a.pz, a.vx, a.vy, a.vz);
+  }
   static __device__ __forceinline__ void finish(const SymArgs &a, int i,
+                                                const Own &p,
                                                 const float (&f)[ACC]) {
-    integrate_ref(a.c, i, f[0], f[1], f[2], a.px, a.py, a.pz, a.vx, a.vy,
-                  a.vz, a.nx, a.ny, a.nz);
+    integrate_loaded(a.c, i, p, f[0], f[1], f[2], a.vx, a.vy, a.vz, a.nx, a.ny,
+                     a.nz);
   }
 };
 
@@ -259,10 +266,15 @@ struct KahanForceRule {
     for (int e = 0; e < 3; ++e) kahan_value(f, e, v[3 + e] - v[e]);
   }
 
+  using Own = Particle;
+  static __device__ __forceinline__ Own own(const SymArgs &a, int i) {
+    return load_particle(i, a.px, a.py, a.pz, a.vx, a.vy, a.vz);
+  }
   static __device__ __forceinline__ void finish(const SymArgs &a, int i,
+                                                const Own &p,
                                                 const float (&f)[ACC]) {
-    integrate_ref(a.c, i, f[0] - f[3], f[1] - f[4], f[2] - f[5], a.px, a.py,
-                  a.pz, a.vx, a.vy, a.vz, a.nx, a.ny, a.nz);
+    integrate_loaded(a.c, i, p, f[0] - f[3], f[1] - f[4], f[2] - f[5], a.vx,
+                     a.vy, a.vz, a.nx, a.ny, a.nz);
   }
 };
 
@@ -348,18 +360,34 @@ struct AdjointRule : PlainPartials<FUSED ? 6 : 3> {
   }
 
   // lx = lx' + dt G sum,  lv = damping g; fused: the forward step too.
+  struct Own {
+    float lx[3], lv[3];
+    Particle p; // fused only
+  };
+  static __device__ __forceinline__ Own own(const SymArgs &a, int i) {
+    Own o;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      o.lx[c] = a.lxn[c][i];
+      o.lv[c] = a.lvn[c][i];
+    }
+    if constexpr (FUSED)
+      o.p = load_particle(i, a.px, a.py, a.pz, a.vx, a.vy, a.vz);
+    return o;
+  }
   static __device__ __forceinline__ void finish(const SymArgs &a, int i,
+                                                const Own &o,
                                                 const float (&f)[ACC]) {
     const float cG = a.c.dt * a.c.G;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const float g = __builtin_fmaf(a.c.dt, a.lxn[c][i], a.lvn[c][i]);
-      a.lx[c][i] = __builtin_fmaf(cG, f[c], a.lxn[c][i]);
+      const float g = __builtin_fmaf(a.c.dt, o.lx[c], o.lv[c]);
+      a.lx[c][i] = __builtin_fmaf(cG, f[c], o.lx[c]);
       a.lv[c][i] = a.c.damping * g;
     }
     if constexpr (FUSED)
-      integrate_ref(a.c, i, f[3], f[4], f[5], a.px, a.py, a.pz, a.vx, a.vy,
-                    a.vz, a.nx, a.ny, a.nz);
+      integrate_loaded(a.c, i, o.p, f[3], f[4], f[5], a.vx, a.vy, a.vz, a.nx,
+                       a.ny, a.nz);
   }
 };
 
@@ -417,13 +445,31 @@ __device__ __forceinline__ void run_sum(float (&f)[R::ACC], int rows,
   const int k0 = run * len / RUNS, k1 = (run + 1) * len / RUNS;
 #pragma unroll
   for (int e = 0; e < R::ACC; ++e) f[e] = 0.0f;
-  if (k0 < rows)
-    sum_partials<R, false>(
-        f, min(k1, rows) - k0, [&](int k) { return row_at(k0 + k); }, stride);
-  const int r0 = max(k0, rows) - rows, r1 = k1 - rows;
-  if (r1 > r0)
-    sum_partials<R, true>(
-        f, r1 - r0, [&](int k) { return reac_at(r0 + k); }, stride);
+  if constexpr (RUNS == 1) { // many partials: no test inside a group of loads
+    if (k0 < rows)
+      sum_partials<R, false>(
+          f, min(k1, rows) - k0, [&](int k) { return row_at(k0 + k); }, stride);
+    const int r0 = max(k0, rows) - rows, r1 = k1 - rows;
+    if (r1 > r0)
+      sum_partials<R, true>(
+          f, r1 - r0, [&](int k) { return reac_at(r0 + k); }, stride);
+  } else { // few: rows and reactions in the same groups of loads, less code
+#pragma unroll 1
+    for (int k = k0; k < k1; k += kInFlight) {
+      float v[kInFlight][R::ACC];
+#pragma unroll
+      for (int u = 0; u < kInFlight; ++u)
+        if (k + u < k1)
+          R::fetch(v[u], k + u < rows ? row_at(k + u) : reac_at(k + u - rows),
+                   stride);
+#pragma unroll
+      for (int u = 0; u < kInFlight; ++u)
+        if (k + u < k1) {
+          if (k + u < rows) R::add_v(f, v[u]);
+          else R::sub_v(f, v[u]);
+        }
+    }
+  }
 }
 
 // First group: f (run 0's sum) plus runs 1 .. RUNS-1 in order.  A run's
@@ -753,19 +799,31 @@ __device__ __forceinline__ int item_row(long long it, int ts, int L) {
   return lo;
 }
 
+// Row of item `it` where rows hold m, m - 1, .. 1 items: counted from the end,
+// the largest k with k (k + 1) / 2 <= r.  The root is off by one at most (it
+// is under 2^17 and rounded to 24 bits).  item_row's search took 800
+// instructions before the first load, in every workgroup at the same time.
+__device__ __forceinline__ int triangle_row(unsigned it, int m) {
+  const unsigned r = (unsigned)((long long)m * (m + 1) / 2) - 1 - it;
+  int k = (int)((__builtin_sqrtf(8.0f * (float)r + 1.0f) - 1.0f) * 0.5f);
+  if ((long long)k * (k + 1) / 2 > r) --k;
+  if ((long long)(k + 1) * (k + 2) / 2 <= r) ++k;
+  return __builtin_amdgcn_readfirstlane(m - 1 - k);
+}
+
 // Work item of a launch -> super-tile ga, its chunk c (row partial
 // row_first(ga) + c).  With one super-tile per item the diagonal pairs, the
 // shorter ones, come last: they fill the last round.
-__device__ __forceinline__ void sym_item(long long it, int ts, int L, int &ga,
+__device__ __forceinline__ void sym_item(unsigned it, int ts, int L, int &ga,
                                          int &c) {
   if (L == 1) {
-    const long long pairs = (long long)ts * (ts - 1) / 2;
+    const unsigned pairs = (unsigned)((long long)ts * (ts - 1) / 2);
     if (it >= pairs) {
       ga = (int)(it - pairs);
       c = 0;
     } else { // rows of lengths ts - 1, .. 1
-      ga = item_row(it, ts - 1, 1);
-      c = (int)(it - row_first(ga, ts - 1, 1)) + 1;
+      ga = triangle_row(it, ts - 1);
+      c = (int)(it - (unsigned)row_first(ga, ts - 1, 1)) + 1;
     }
   } else {
     ga = item_row(it, ts, L);
@@ -797,17 +855,27 @@ constexpr int kTileRuns = 4; // runs per particle, tile-pair finalize
 template <class R, int ST, int RUNS>
 __global__ __launch_bounds__(256) void sym_finalize(SymArgs a) {
   constexpr int PW = 256 / RUNS; // particles per workgroup
+  static_assert(ST % PW == 0 && PW % 64 == 0, "one super-tile per workgroup, "
+                                              "one run per wave");
   __shared__ float red[RUNS > 1 ? R::ACC : 1][256];
-  const int i = blockIdx.x * PW + threadIdx.x % PW;
+  // uniform: the indices of the partials are scalar arithmetic (per-lane
+  // indices with 64-bit divisions were 300 instructions before the first
+  // load; with that, the work items' search and the particle's own loads moved
+  // here, a step takes 1 us less: n = 4097 12.9 -> 11.8, 12800 38.0 -> 37.1)
+  const int base = blockIdx.x * PW, g = base / ST;
+  const int run =
+      RUNS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / PW) : 0;
+  const int i = base + threadIdx.x % PW, o = base % ST + threadIdx.x % PW;
   const bool live = i < a.n;
   if (RUNS == 1 && !live) return;
+  typename R::Own own = {}; // in flight with the partials
+  if (run == 0 && live) own = R::own(a, i);
   float f[R::ACC];
   if (live) {
-    const int g = i / ST, o = i % ST;
     const int ts = a.ts, L = a.chunk;
     const long long first = row_first(g, ts, L);
     run_sum<R, RUNS>(
-        f, (ts - g + L - 1) / L, g, threadIdx.x / PW,
+        f, L == 1 ? ts - g : (ts - g + L - 1) / L, g, run,
         [&](int c) { return a.fpart + (size_t)(first + c) * (R::ACC * ST) + o; },
         [&](int ga) {
           return a.spart + (size_t)pair_slot(ga, g, ts) * (R::ACC * ST) + o;
@@ -817,7 +885,7 @@ __global__ __launch_bounds__(256) void sym_finalize(SymArgs a) {
 #pragma unroll
     for (int e = 0; e < R::ACC; ++e) f[e] = 0.0f;
   }
-  if (combine_runs<R, RUNS>(f, red) && live) R::finish(a, i, f);
+  if (combine_runs<R, RUNS>(f, red) && live) R::finish(a, i, own, f);
 }
 
 // ---- banded launches (n past the single-launch limit) ----------------------
@@ -926,7 +994,7 @@ __global__ __launch_bounds__(256) void sym_band_finish(SymArgs a) {
   float f[R::ACC];
 #pragma unroll
   for (int e = 0; e < R::ACC; ++e) f[e] = a.acc3[(size_t)e * a.n + i];
-  R::finish(a, i, f);
+  R::finish(a, i, R::own(a, i), f);
 }
 
 // ---- many independent systems (batched persistent launch) ----------------
@@ -1051,7 +1119,7 @@ __global__ __launch_bounds__(256) void sym_batch_finalize(SymBatchArgs b) {
                R::ACC * ST;
       },
       ST);
-  R::finish(a, li, f);
+  R::finish(a, li, R::own(a, li), f);
 }
 
 using KernelFn = void (*)(SymArgs);
@@ -1061,12 +1129,31 @@ using KernelFn = void (*)(SymArgs);
 struct SymShape {
   int st, threads, runs;
   KernelFn pairs, finalize;
+  int even_lds; // see even_rounds (0: not for this shape)
 };
+
+// Kahan sums and the fused adjoint take 114 to 124 VGPRs with 4 targets per
+// lane: four workgroups fit a CU.  Where a CU gets five, the fifth would run
+// alone, one wave per SIMD with nothing to issue beside it; with LDS for three
+// they run as 3 + 2.  Us per step, 4 + 1 / 3 + 2, Kahan and fused: n = 11520
+// 62.9 / 62.5 and 67.2 / 66.2, 12288 65.3 / 63.8 and 69.3 / 67.8, 12800 70.3 /
+// 65.0 and 74.5 / 69.5.  With four per CU (11264) 52.9 / 59.8, with six (13056)
+// 72.0 / 75.2, with nine (16640) 103.7 / 105.7; the rules with more workgroups
+// per CU gain nothing.
+constexpr int kCUs = 256;
+constexpr int kThirdOfLds = 160 * 1024 / 3 / 1280 * 1280; // bytes
+
+bool even_rounds(long long blocks) {
+  return blocks > 4 * kCUs && blocks <= 5 * kCUs;
+}
 
 template <class R, int U, int M, int RUNS, int W = (M > 2 ? 8 : 4)>
 constexpr SymShape sym_shape() {
   constexpr int ST = 64 * U * M;
-  return {ST, 64 * W, RUNS, sym_kernel<R, U, M, W>, sym_finalize<R, ST, RUNS>};
+  constexpr bool four = U == 4 && R::ACC == 6;
+  constexpr int lds = (int)sizeof(float) * RowShape<R, U, M, W>::LDS_FLOATS;
+  return {ST,   64 * W, RUNS, sym_kernel<R, U, M, W>, sym_finalize<R, ST, RUNS>,
+          four ? kThirdOfLds - lds : 0};
 }
 
 // Targets per lane of a tile-pair shape: `unroll` particles per lane and
@@ -1246,7 +1333,8 @@ int launch_sym(const SymShape *sh, SymArgs &a, int unroll, int chunk, int n,
   void *args[] = {&a};
   int r = hip_check(hipLaunchKernel(reinterpret_cast<const void *>(sh->pairs),
                                     dim3((unsigned)blocks), dim3(sh->threads),
-                                    args, 0, stream),
+                                    args, even_rounds(blocks) ? sh->even_lds : 0,
+                                    stream),
                     "symmetric pair launch");
   if (r) return r;
   const int per_block = 256 / sh->runs;
