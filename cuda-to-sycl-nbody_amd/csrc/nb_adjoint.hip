@@ -26,7 +26,8 @@
 // formed while the tile is staged).  Optional source split with a finalize
 // kernel.  Built with -ffp-contract=off; fused ops are explicit.
 
-#include "nb_internal.hpp"
+#include "nb_pairs.hpp"
+#include "nb_small.hpp"
 
 namespace nb {
 namespace {
@@ -109,35 +110,42 @@ __device__ __forceinline__ void load_g(const AdjArgs &a, int j, float &gx,
   gz = __builtin_fmaf(dt, a.lxn[2][j], a.lvn[2][j]);
 }
 
+// What the outputs of a particle need besides its sums.
+struct AdjOwn {
+  float lx[3], lv[3];
+  Particle p; // fused only
+};
+
+template <bool FUSED>
+__device__ __forceinline__ AdjOwn adj_own(const AdjArgs &a, int i) {
+  AdjOwn o;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    o.lx[c] = a.lxn[c][i];
+    o.lv[c] = a.lvn[c][i];
+  }
+  if constexpr (FUSED)
+    o.p = load_particle(i, a.px, a.py, a.pz, a.vx, a.vy, a.vz);
+  return o;
+}
+
 // Writes the outputs of target i from its accumulated sums.
 template <bool FUSED>
-__device__ __forceinline__ void adj_epilogue(const AdjArgs &a, int i, float gx,
-                                             float gy, float gz, float ax,
+__device__ __forceinline__ void adj_epilogue(const AdjArgs &a, int i,
+                                             const AdjOwn &o, float ax,
                                              float ay, float az, float fx,
                                              float fy, float fz) {
   const float cG = a.c.dt * a.c.G;
   const float acc[3] = {ax, ay, az};
-  const float g[3] = {gx, gy, gz};
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    a.lx[c][i] = __builtin_fmaf(cG, acc[c], a.lxn[c][i]);
-    a.lv[c][i] = a.c.damping * g[c];
+    const float g = __builtin_fmaf(a.c.dt, o.lx[c], o.lv[c]);
+    a.lx[c][i] = __builtin_fmaf(cG, acc[c], o.lx[c]);
+    a.lv[c][i] = a.c.damping * g;
   }
-  if constexpr (FUSED) {
-    // forward step in the reference's rounding order (src/simulator.cu:214-228)
-    float vx = a.vx[i] * a.c.damping;
-    float vy = a.vy[i] * a.c.damping;
-    float vz = a.vz[i] * a.c.damping;
-    vx = vx + (fx * a.c.dt) * a.c.G;
-    vy = vy + (fy * a.c.dt) * a.c.G;
-    vz = vz + (fz * a.c.dt) * a.c.G;
-    a.vx[i] = vx;
-    a.vy[i] = vy;
-    a.vz[i] = vz;
-    a.nx[i] = a.px[i] + vx * a.c.dt;
-    a.ny[i] = a.py[i] + vy * a.c.dt;
-    a.nz[i] = a.pz[i] + vz * a.c.dt;
-  }
+  if constexpr (FUSED) // the forward step in the reference's rounding order
+    integrate_loaded(a.c, i, o.p, fx, fy, fz, a.vx, a.vy, a.vz, a.nx, a.ny,
+                     a.nz);
 }
 
 template <int BLOCK, int U, int TILE, bool SKIP, bool FUSED, bool SPLIT>
@@ -235,7 +243,7 @@ __global__ __launch_bounds__(BLOCK) void adj_kernel(AdjArgs a) {
       p[4 * nn + i] = T.fy[k];
       p[5 * nn + i] = T.fz[k];
     } else {
-      adj_epilogue<FUSED>(a, i, T.gx[k], T.gy[k], T.gz[k], T.ax[k], T.ay[k],
+      adj_epilogue<FUSED>(a, i, adj_own<FUSED>(a, i), T.ax[k], T.ay[k],
                           T.az[k], T.fx[k], T.fy[k], T.fz[k]);
     }
   }
@@ -252,9 +260,105 @@ __global__ __launch_bounds__(256) void adj_finalize(AdjArgs a) {
 #pragma unroll
     for (int c = 0; c < 6; ++c) s[c] = s[c] + p[c * nn + i];
   }
-  float gx, gy, gz;
-  load_g(a, i, gx, gy, gz);
-  adj_epilogue<FUSED>(a, i, gx, gy, gz, s[0], s[1], s[2], s[3], s[4], s[5]);
+  adj_epilogue<FUSED>(a, i, adj_own<FUSED>(a, i), s[0], s[1], s[2], s[3], s[4],
+                      s[5]);
+}
+
+// One launch for small systems: as fwd_small_kernel (nb_forward.hip), whose
+// order of sources and sums it keeps, so that the fused forward part has its
+// bits.  Sources are read two at a time (each is nine loads).  Latency, as
+// there: 4.0 us at n = 1000 (fused 4.9; tile pairs and their finalize 8.7 and
+// 10.2).
+template <int U, bool SKIP, bool FUSED>
+__global__ __launch_bounds__(kSmallBlock) void adj_small_kernel(AdjArgs a) {
+  constexpr int NT = 4 * U; // targets per workgroup
+  constexpr int WAVES = kSmallBlock / 64;
+  constexpr int NV = FUSED ? 6 : 3;
+  static_assert(WAVES == kSmallLanes, "one lane of a row per wave's sum");
+  __shared__ float sums[NV][NT][WAVES];
+  const int n = a.n;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = lane >> 4, sl = lane & 15;
+  const int first = blockIdx.x * NT;
+
+  // lane 0 of row r (of the workgroup) writes target first + r
+  const int fin = threadIdx.x >> 4;
+  const bool owner = sl == 0 && fin < NT && first + fin < n;
+  AdjOwn own = {};
+  if (owner) own = adj_own<FUSED>(a, first + fin);
+
+  AdjTargets<U, SKIP, FUSED> T;
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    const int i = first + row * U + k, ic = min(i, n - 1);
+    T.idx[k] = i;
+    T.x[k] = a.px[ic];
+    T.y[k] = a.py[ic];
+    T.z[k] = a.pz[ic];
+    load_g(a, ic, T.gx[k], T.gy[k], T.gz[k]);
+    T.ax[k] = T.ay[k] = T.az[k] = 0.0f;
+    T.fx[k] = T.fy[k] = T.fz[k] = 0.0f;
+  }
+
+  const int s0 = wave * kSmallLanes + sl;
+  constexpr int B = 2, PASS = kSmallStride * B;
+  float P[B][3], LX[B][3], LV[B][3];
+  auto fetch = [&](int b) {
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      const int j = min(b + q * kSmallStride + s0, n - 1);
+      P[q][0] = a.px[j];
+      P[q][1] = a.py[j];
+      P[q][2] = a.pz[j];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        LX[q][c] = a.lxn[c][j];
+        LV[q][c] = a.lvn[c][j];
+      }
+    }
+  };
+  fetch(0);
+  for (int b = 0; b < n; b += PASS) {
+    float x[B][3], g[B][3];
+#pragma unroll
+    for (int q = 0; q < B; ++q)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        x[q][c] = P[q][c];
+        g[q][c] = __builtin_fmaf(a.c.dt, LX[q][c], LV[q][c]);
+      }
+    if (b + PASS < n) fetch(b + PASS);
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      const int j = b + q * kSmallStride + s0;
+      if (j < n)
+        T.one(x[q][0], x[q][1], x[q][2], g[q][0], g[q][1], g[q][2], j,
+              a.c.eps);
+    }
+  }
+
+  float none = 0.0f;
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    float *v[6] = {&T.ax[k], &T.ay[k], &T.az[k],
+                   &T.fx[k], &T.fy[k], &T.fz[k]};
+#pragma unroll
+    for (int m = 0; m < NV; ++m) {
+      row_sum<false>(*v[m], none);
+      if (sl == 0) sums[m][row * U + k][wave] = *v[m];
+    }
+  }
+  __syncthreads();
+  if (wave >= U) return; // NT rows of 16 lanes are U waves
+  float f[6] = {};
+#pragma unroll
+  for (int m = 0; m < NV; ++m) {
+    f[m] = sums[m][fin][sl];
+    row_sum<false>(f[m], none);
+  }
+  if (owner)
+    adj_epilogue<FUSED>(a, first + fin, own, f[0], f[1], f[2], f[3], f[4],
+                        f[5]);
 }
 
 using AdjFn = void (*)(AdjArgs);
@@ -271,6 +375,15 @@ AdjFn adj_shape(bool skip, bool fused, bool split) {
                           : adj_kernel<B, U, T, false, true, false>;
   return split ? adj_kernel<B, U, T, false, false, true>
                : adj_kernel<B, U, T, false, false, false>;
+}
+
+template <int U>
+AdjFn adj_small(bool skip, bool fused) {
+  if (skip)
+    return fused ? adj_small_kernel<U, true, true>
+                 : adj_small_kernel<U, true, false>;
+  return fused ? adj_small_kernel<U, false, true>
+               : adj_small_kernel<U, false, false>;
 }
 
 struct AdjShape {
@@ -299,6 +412,7 @@ const FwdConfig kAdjConfigs[] = {
     {256, 2, 128, 1, SCHEME_SYMMETRIC_TILES},
     {256, 2, 512, 1, SCHEME_SYMMETRIC}, {256, 2, 512, 2, SCHEME_SYMMETRIC},
     {256, 4, 1024, 4, SCHEME_SYMMETRIC}, {256, 2, 512, 4, SCHEME_SYMMETRIC},
+    {kSmallBlock, 1, 1024, 1}, // one launch (adj_small_kernel)
 };
 constexpr int kNumAdj = sizeof(kAdjConfigs) / sizeof(kAdjConfigs[0]);
 
@@ -315,13 +429,16 @@ int adjoint_config_count() { return kNumAdj; }
 const FwdConfig &adjoint_config(int cfg) { return kAdjConfigs[cfg]; }
 
 int adjoint_default_config(size_t n, bool skip) {
-  // Measured on MI355X (disk ICs), adjoint / fused us (device time).  Tile
-  // pairs, 2 per lane: n = 64 7.3 / 8.6 (target-sharded 256 x 1 split 2 7.1 /
-  // 8.1), 300 8.9 / 10.5 (20.7 / 23.9), 4097 17 / 21 (63 / 72), 12000 57 / 76
-  // (super-tiles of 512, 1 per item 71 / 89), 24000 162 / 215 (176 / 229),
-  // 30720 264.1 / 350.4 (274.5 / 359.1), 34000 321.8 / 428.6 (313.3 / 407.4).
-  // Super-tiles of 512, 1 / 2 per item: 65536 1041 / 1369 vs 1052 / 1411 (tile pairs 1099 / 1490), 100000 2371 / 3160 vs
-  // 2360 / 3124, 262144 16154 / 21434 vs 15812 / 21092 (super-tiles of 1024:
+  // Measured on MI355X (disk ICs), adjoint / fused us (device time).  One
+  // launch, and tile pairs, 2 per lane: n = 32 2.9 / 3.4 and 6.8 / 7.8
+  // (target-sharded 256 x 1 split 2 5.4 / 5.7), 1000 4.0 / 4.9 and 8.7 / 10.2
+  // (58 / 67), 2000 6.9 / 8.2 and 9.2 / 10.9, 2500 11.7 / 13.4 and 9.7 / 11.5,
+  // 4000 17.1 / 19.2 and 15.1 / 18.4.  Tile pairs: 4097 15.1 / 19.1 (63 / 72),
+  // 12800 53.5 / 70.6, 24000 162 / 215 (super-tiles of 512, 1 per item 176 /
+  // 229), 30720 264.1 / 350.4 (274.5 / 359.1), 34000 321.8 / 428.6 (313.3 /
+  // 407.4).
+  // Super-tiles of 512, 1 / 2 per item: 65536 1041 / 1369 vs 1052 / 1411 (tile
+  // pairs 1099 / 1490), 100000 2371 / 3160 vs 2360 / 3124, 262144 16154 / 21434 vs 15812 / 21092 (super-tiles of 1024:
   // 16461 / 22713 on a card where 2 per item took 16509 / 21775).  Best
   // target-sharded at 262144 31.5 / 39.0 ms.  Past 2^18 four super-tiles per
   // item and bands of source super-tiles.
@@ -330,11 +447,10 @@ int adjoint_default_config(size_t n, bool skip) {
   if (n <= kSymMaxParticles) { // skip or not: self pairs masked in-kernel
     if (n >= 98304) return 20; // super-tile pairs, 2 per lane, 2 per item
     if (n >= 32768) return 19; // super-tile pairs, 2 per lane, 1 per item
-    if (n >= 96) return 18;    // tile pairs, 2 per lane
+    if (n > 2048) return 18;   // tile pairs, 2 per lane
+    return 23;                 // one launch
   }
-  if (n >= (size_t)1 << 17) return 8; // 256 x 1, split 2
-  if (n < 4096) return 8;
-  return 9;                           // 256 x 2, split 4
+  return 8; // 256 x 1, split 2
 }
 
 size_t adjoint_scratch_bytes(int cfg, size_t n) {
@@ -363,7 +479,12 @@ int launch_adjoint(const StepConsts &c, bool skip, bool fused, int cfg,
                               fc.scheme == SCHEME_SYMMETRIC_TILES, pos, lxn, lvn,
                               lx, lv, vel, nxt, n, scratch, stream);
   }
-  AdjFn fn = find_adj(fc, skip, fused);
+  const bool small = fc.block == kSmallBlock;
+  const int per_row = small ? small_targets(n) : 0;
+  AdjFn fn = !small         ? find_adj(fc, skip, fused)
+             : per_row == 1 ? adj_small<1>(skip, fused)
+             : per_row == 2 ? adj_small<2>(skip, fused)
+                            : adj_small<4>(skip, fused);
   if (!fn) return set_error(NB_ERR_UNSUPPORTED, "no adjoint kernel for shape");
   if (fc.split > 1 && !scratch)
     return set_error(NB_ERR_INVALID_ARG, "split launch needs scratch");
@@ -391,7 +512,7 @@ int launch_adjoint(const StepConsts &c, bool skip, bool fused, int cfg,
   const int per_chunk = (n + fc.split - 1) / fc.split;
   a.jchunk = ((per_chunk + fc.tile - 1) / fc.tile) * fc.tile;
   a.c = c;
-  const int targets = fc.block * fc.unroll;
+  const int targets = small ? 4 * per_row : fc.block * fc.unroll;
   dim3 grid((n + targets - 1) / targets, fc.split);
   void *args[] = {&a};
   int st = hip_check(hipLaunchKernel(reinterpret_cast<const void *>(fn), grid,

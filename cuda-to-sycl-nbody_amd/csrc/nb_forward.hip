@@ -19,6 +19,7 @@
 // sum separately, as written in the reference.
 
 #include "nb_pairs.hpp"
+#include "nb_small.hpp"
 
 
 namespace nb {
@@ -106,44 +107,6 @@ __global__ __launch_bounds__(256) void fwd_finalize(FwdArgs a) {
 // the lanes that integrate have loaded their particles at the start.
 // Device time at n = 1000 3.4 us, 4000 8.9 (split shapes and a second kernel:
 // 23.8, 24.8); the launch and two dependent trips to L2 are about 3 of it.
-
-constexpr int kSmallBlock = 1024;
-constexpr int kSmallLanes = 16;                         // source lanes per row
-constexpr int kSmallStride = kSmallBlock / 64 * kSmallLanes; // sources per pass
-constexpr int kSmallBatch = 4;
-
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
-                                         0xf, 0xf, false));
-}
-
-// (s, c) stands for s - c.  TwoSum keeps the rounding of s + s' in c.
-__device__ __forceinline__ void meet(float &s, float &c, float s2, float c2) {
-  const float t = s + s2;
-  const float b = t - s;
-  const float err = (s - (t - b)) + (s2 - b);
-  c = (c + c2) - err;
-  s = t;
-}
-
-template <bool KAHAN, int CTRL>
-__device__ __forceinline__ void row_step(float &s, float &c) {
-  if constexpr (KAHAN)
-    meet(s, c, dpp<CTRL>(s), dpp<CTRL>(c));
-  else
-    s = s + dpp<CTRL>(s);
-}
-
-// Sum over a row of 16 lanes, in every lane of it (row_ror 8, 4, 2, 1).
-template <bool KAHAN>
-__device__ __forceinline__ void row_sum(float &s, float &c) {
-  row_step<KAHAN, 0x128>(s, c);
-  row_step<KAHAN, 0x124>(s, c);
-  row_step<KAHAN, 0x122>(s, c);
-  row_step<KAHAN, 0x121>(s, c);
-}
 
 template <int U, int MODE>
 __global__ __launch_bounds__(kSmallBlock) void fwd_small_kernel(FwdArgs a) {
@@ -308,12 +271,6 @@ KernelFn find_kernel(const FwdConfig &c, int mode) {
       return s.get(mode, c.split > 1);
   return nullptr;
 }
-
-// Targets per row of the one-launch shape: as few as leave one workgroup for
-// each of the 256 CUs.  1 / 2 / 4 targets, us: n = 1000 3.4 / 3.6 / 4.3, 1500
-// 4.7 / 4.3 / 5.4, 2000 5.1 / 4.6 / 5.8, 3000 8.1 / 7.7 / 7.5, 4000 11.7 / 9.2
-// / 8.9.
-int small_targets(int n) { return n <= 1024 ? 1 : n <= 2048 ? 2 : 4; }
 
 } // namespace
 
