@@ -5,6 +5,8 @@
 //   F_i = sum_{j != i} r_ij * rsqrt(d^3),  r_ij = x_j - x_i,  d = |r_ij|^2 + eps
 //   v_i <- v_i * damping;  v_i <- v_i + (F_i * dt) * G;  x'_i = x_i + v_i * dt
 //
+// Below 4096 particles one launch does the step (fwd_small_kernel); the
+// symmetric shapes above are in nb_sym.hip.  The target-sharded shapes:
 // Mapping (one workgroup = BLOCK threads x U targets):
 //   * target i's position and force accumulator live in VGPRs, U per thread
 //     (i = base + k * BLOCK + lane, so global loads/stores stay coalesced);
@@ -241,7 +243,9 @@ const ShapeEntry kShapes[] = {
 // Compiled launch shapes: {block, unroll, tile, split[, scheme]}.  Index 0
 // must stay the unsplit 256 x 1 shape (a valid choice for every n).  The
 // symmetric shapes (nb_sym.hip) are {256, particles per lane, super-tile,
-// super-tiles per work item}.
+// super-tiles per work item}, where 256 x particles per lane is the super-tile:
+// the workgroups have 256 threads, 512 with 8 per lane and for tile pairs of 2
+// per lane below 3328 particles.
 const FwdConfig kConfigs[] = {
     {256, 1, 1024, 1}, {256, 1, 1024, 2}, {256, 1, 1024, 4},
     {256, 1, 1024, 8}, {256, 2, 1024, 1}, {256, 2, 1024, 2},

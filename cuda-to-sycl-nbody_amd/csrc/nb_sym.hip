@@ -18,7 +18,7 @@
 // target-sharded kernels.
 //
 // Particles are grouped in super-tiles of ST; a work item is one workgroup (4
-// waves) and a chunk of one row of the super-tile pair triangle: super-tile
+// or 8 waves) and a chunk of one row of the super-tile pair triangle: super-tile
 // GA against super-tiles GB in [GB0, GB1), GB >= GA.  Each item writes the
 // targets' sums over its chunk as one row partial and, per pair with GB > GA,
 // the (negated) reaction sums of GB's particles.  A finalize kernel sums, per
@@ -1162,13 +1162,15 @@ constexpr SymShape sym_shape() {
 // at a time (super-tiles of 128, two waves per set of sources: four times the
 // workgroups); from there two at a time (4 targets per lane, half the LDS
 // traffic and partials per pair term).  Both sides, us per step, device time
-// (forward / Kahan / adjoint / fused): n = 4097 13.4 / 20 / 17 / 21 vs 19.4 /
-// 28 / 24 / 31, 9000 27.5 / 46.7 / 38.6 / 50.9 vs 27.2 / 47.3 / 41.1 / 52.7,
-// 12000 42.1 / 71.3 / 59.1 / 78.9 vs 38.2 / 67.2 / 57.0 / 75.9.
+// (forward / Kahan / adjoint / fused): n = 4097 11.8 / 17.7 / 15.1 / 19.1 vs
+// 17.9 / 26.6 / 23.7 / 28.5, 9000 26.8 / 42.8 / 35.5 / 46.7 vs 25.5 / 44.2 /
+// 38.5 / 49.4, 9728 29.9 / 48.6 / 39.9 / 52.8 vs 25.8 / 44.8 / 36.6 / 47.2,
+// 11000 35.5 / 58.6 / 48.0 / 64.6 vs 30.9 / 52.5 / 46.4 / 60.7.
 // Below kTileWide particles 8 waves share the 128 x 128 pairs, each a quarter
 // of a set's steps: with fewer pairs than SIMDs the step is the latency of
-// one wave (n = 1000 8.9 / 11.0 / 10.0 / 11.9 vs 10.2 / 12.9 / 12.0 / 14.1,
-// 4097 13.8 / 20.7 / 17.4 / 21.5 vs 13.4 / 20.0 / 17.1 / 21.3).
+// one wave (2100 8.8 / 10.3 / 10.7 / 12.0 vs 9.6 / 12.6 / 11.2 / 13.0, 3000
+// 10.1 / 13.8 / 11.5 / 14.4 vs 10.2 / 13.3 / 12.4 / 14.6, 4097 12.2 / 18.2 /
+// 15.1 / 19.1 vs 11.8 / 17.7 / 15.1 / 19.1).
 constexpr size_t kTilePairRows = 9728;
 constexpr size_t kTileWide = 3328;
 

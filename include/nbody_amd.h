@@ -232,9 +232,12 @@ int nb_forward_default_config(const nb_params *p, size_t n, int acc);
  *                        scratch growing as n^2 (0.4 GB at n = 2^18 with 8
  *                        per lane, 16 GB at 2^21, at most 8 GB per band,
  *                        twice that with Kahan sums);
- *                        work item = a pair of 4-tile super-tiles;
- *   NB_SCHEME_SYMMETRIC_TILES  the same with one tile pair per wave, for
+ *                        work item = a pair of super-tiles (workgroups of
+ *                        256 threads, 512 with 8 per lane);
+ *   NB_SCHEME_SYMMETRIC_TILES  the same with pairs of small tiles, for
  *                        small n (n <= 2^17).
+ * A target-sharded shape of block 1024 does the step in one launch with no
+ * scratch: the default below 4096 particles (adjoint: up to 2048).
  * Returns the scheme, or -1 (and sets nb_last_error) for a bad index. */
 #define NB_SCHEME_TARGETS 0
 #define NB_SCHEME_SYMMETRIC 1
