@@ -453,6 +453,14 @@ int adjoint_default_config(size_t n, bool skip) {
   return 8; // 256 x 1, split 2
 }
 
+bool adjoint_one_launch(int cfg) {
+  return kAdjConfigs[cfg].block == kSmallBlock;
+}
+
+int adjoint_overlap_config(size_t n) {
+  return n < 1024 ? 8 : 18; // 256 x 1, split 2; tile pairs, 2 per lane
+}
+
 size_t adjoint_scratch_bytes(int cfg, size_t n) {
   const FwdConfig &c = kAdjConfigs[cfg];
   if (c.scheme != SCHEME_TARGETS) { // either variant (3 or 6 sums)

@@ -649,7 +649,15 @@ int check_forward_dev(const nb_params *p, const float *px, const float *py,
     return set_error(NB_ERR_INVALID_ARG,
                      "positions and next positions must not alias");
   *mode = pair_mode(p->calc_method, acc, p->dist_eps);
-  if (*cfg < 0) *cfg = forward_default_config(n, *mode);
+  const bool chosen = *cfg < 0;
+  if (chosen) *cfg = forward_default_config(n, *mode);
+  if (forward_one_launch(*cfg) &&
+      any_overlap({vx, vy, vz, nx, ny, nz}, {px, py, pz}, n)) {
+    if (!chosen)
+      return set_error(NB_ERR_INVALID_ARG,
+                       "one-launch shape: outputs must not overlap positions");
+    *cfg = forward_overlap_config();
+  }
   return NB_OK;
 }
 

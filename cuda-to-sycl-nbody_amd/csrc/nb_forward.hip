@@ -346,6 +346,11 @@ int forward_default_config(size_t n, int mode) {
   return 30;                           // 128 x 1, tile 512, split 8
 }
 
+bool forward_one_launch(int cfg) { return kConfigs[cfg].block == kSmallBlock; }
+
+// Every mode and every n below 4096, where one launch is the default: 24 us.
+int forward_overlap_config() { return 30; } // 128 x 1, tile 512, split 8
+
 int forward_launches(int cfg) {
   const FwdConfig &c = kConfigs[cfg];
   return c.scheme == SCHEME_TARGETS && c.split == 1 ? 1 : 2;

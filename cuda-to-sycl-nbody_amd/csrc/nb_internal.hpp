@@ -67,6 +67,25 @@ int forward_config_count();
 const FwdConfig &forward_config(int cfg);
 // Library's launch shape for n particles in pair mode `mode` (MODE_*).
 int forward_default_config(size_t n, int mode);
+// One-launch shapes write a step's outputs while other workgroups still read
+// its sources.  A call whose outputs overlap its sources takes this shape of
+// two launches in place of a one-launch default.
+bool forward_one_launch(int cfg);
+int forward_overlap_config();
+
+// True if an array of `outs` shares memory with one of `srcs` (n floats each).
+template <size_t O, size_t S>
+inline bool any_overlap(const float *const (&outs)[O],
+                        const float *const (&srcs)[S], size_t n) {
+  const uintptr_t bytes = n * sizeof(float);
+  for (const float *o : outs)
+    for (const float *s : srcs) {
+      const uintptr_t a = reinterpret_cast<uintptr_t>(o);
+      const uintptr_t b = reinterpret_cast<uintptr_t>(s);
+      if ((a > b ? a - b : b - a) < bytes) return true;
+    }
+  return false;
+}
 
 // Largest particle count of the symmetric scheme (its partial buffers grow
 // as n^2: 4.0 GB at 2^20 with 8 particles per lane and 4-tile chunks).
@@ -204,6 +223,8 @@ __host__ __device__ inline bool self_term_vanishes(float eps) {
 int adjoint_config_count();
 const FwdConfig &adjoint_config(int cfg);
 int adjoint_default_config(size_t n, bool skip);
+bool adjoint_one_launch(int cfg); // as forward_one_launch
+int adjoint_overlap_config(size_t n);
 size_t adjoint_scratch_bytes(int cfg, size_t n);
 
 // Adjoint of one step at positions pos: reads the cotangents of the step's

@@ -58,7 +58,21 @@ int adjoint_common(const nb_params *p, const nb_vec3 *pos, const nb_vec3 *vel,
       overlaps(lv, lvn) || overlaps(lx, lv) ||
       (fused && (overlaps(nxt, pos) || overlaps(vel, pos))))
     return set_error(NB_ERR_INVALID_ARG, "outputs must not alias inputs");
-  if (cfg < 0) cfg = adjoint_default_config(n, !self_term_vanishes(p->dist_eps));
+  const bool chosen = cfg < 0;
+  if (chosen) cfg = adjoint_default_config(n, !self_term_vanishes(p->dist_eps));
+  if (adjoint_one_launch(cfg)) {
+    const nb_vec3 *const fv = fused ? vel : lx, *const fn = fused ? nxt : lv;
+    if (any_overlap({lx->x, lx->y, lx->z, lv->x, lv->y, lv->z, fv->x, fv->y,
+                     fv->z, fn->x, fn->y, fn->z},
+                    {pos->x, pos->y, pos->z, lxn->x, lxn->y, lxn->z, lvn->x,
+                     lvn->y, lvn->z},
+                    n)) {
+      if (!chosen)
+        return set_error(NB_ERR_INVALID_ARG,
+                         "one-launch shape: outputs must not overlap inputs");
+      cfg = adjoint_overlap_config(n);
+    }
+  }
   const hipStream_t s = static_cast<hipStream_t>(stream);
   ScratchLease scratch; // held until the launches are enqueued
   if ((st = acquire_scratch(adjoint_scratch_bytes(cfg, n), s, scratch))) return st;

@@ -262,7 +262,8 @@ def pack_vec4(soa, w: float = 1.0, stream=None):
 def forward_step(params: NbParams, pos, vel, nxt, n: int | None = None, cfg: int = -1,
                  acc: int = NB_ACC_PLAIN, stream=None) -> None:
     """One stream-ordered step on device tensors: reads pos, updates vel in
-    place, writes nxt (3 tensors each).  stream: a torch.cuda.Stream or None
+    place, writes nxt (3 tensors each).  nxt must not share memory with pos;
+    vel may be rows of pos (cfg=-1 only).  stream: a torch.cuda.Stream or None
     (the current stream)."""
     n = row_length(pos) if n is None else int(n)
     p = row_ptrs(pos, n) or _dev_ptrs(pos, n, "pos")

@@ -40,7 +40,9 @@ def _stream(stream):
 
 def adjoint_step(params: NbParams, pos, lam_x_next, lam_v_next, lam_x, lam_v, cfg: int = -1,
                  stream=None) -> None:
-    """Cotangents of (x_n, v_n) from those of (x_{n+1}, v_{n+1}) at positions pos."""
+    """Cotangents of (x_n, v_n) from those of (x_{n+1}, v_{n+1}) at positions pos.
+    lam_x and lam_v must not share memory with the incoming cotangents or each
+    other; they may be rows of pos (cfg=-1 only, at some cost below 2049)."""
     n = row_length(pos)
     vs = [_vec3(t, n) for t in (pos, lam_x_next, lam_v_next, lam_x, lam_v)]
     check(load().nb_adjoint_step_dev(ctypes.byref(params), *vs, n, cfg,
@@ -49,7 +51,10 @@ def adjoint_step(params: NbParams, pos, lam_x_next, lam_v_next, lam_x, lam_v, cf
 
 def fwd_adjoint_step(params: NbParams, pos, vel, pos_next, lam_x_next, lam_v_next, lam_x, lam_v,
                      cfg: int = -1, stream=None) -> None:
-    """Forward step (vel in place, pos_next written) and adjoint step at pos, one launch."""
+    """Forward step (vel in place, pos_next written) and adjoint step at pos, one
+    launch for the pairs of both.  vel and pos_next must not share memory with
+    pos; they may be rows of the incoming cotangents (cfg=-1 only, as
+    adjoint_step's lam_x and lam_v of pos)."""
     n = row_length(pos)
     vs = [_vec3(t, n) for t in (pos, vel, pos_next, lam_x_next, lam_v_next, lam_x, lam_v)]
     check(load().nb_fwd_adjoint_step_dev(ctypes.byref(params), *vs, n, cfg,

@@ -181,6 +181,9 @@ int nb_sim_destroy(nb_sim *s);
 /* One launch of particle_interaction (src/simulator.cu:186-229):
  *   reads pos (px,py,pz), updates vel (vx,vy,vz) in place, writes the next
  *   positions (nx,ny,nz).  pos and next must not overlap.  n = particle count.
+ *   vel may be rows of pos: cfg = -1 then takes a shape that reads every
+ *   position before it writes (two launches), and the one-launch shape is
+ *   refused.
  * cfg selects a tuned launch shape (-1 = the library's choice for n);
  * acc is NB_ACC_*. */
 int nb_forward_step_dev(const nb_params *p, const float *px, const float *py,
@@ -276,7 +279,11 @@ typedef struct nb_vec3 {
  *   lam_x = lam_x_next + dt * G * sum_{j != k} M_kj (g_j - g_k),
  *   M = K (I - 3 r r^T / d),  d = |r|^2 + eps,  K = d^-3/2,
  * evaluated at positions pos (x_n) in one pass over all pairs.  BRANCH only.
- * lam_x / lam_v must not alias the inputs.  cfg: -1 = library's shape. */
+ * lam_x / lam_v must not share memory with lam_x_next / lam_v_next or each
+ * other (equal rows are refused).  They may be rows of pos, which the call
+ * then overwrites: cfg = -1 takes a shape of two launches, which reads every
+ * input before it writes, and the one-launch shape is refused.
+ * cfg: -1 = library's shape. */
 int nb_adjoint_step_dev(const nb_params *p, const nb_vec3 *pos,
                         const nb_vec3 *lam_x_next, const nb_vec3 *lam_v_next,
                         const nb_vec3 *lam_x, const nb_vec3 *lam_v, size_t n,
@@ -285,7 +292,9 @@ int nb_adjoint_step_dev(const nb_params *p, const nb_vec3 *pos,
 /* The forward step and the adjoint step at the same positions in one
  * launch: vel is updated in place and pos_next written (as
  * nb_forward_step_dev), and the cotangents propagated (as
- * nb_adjoint_step_dev).  The pair quantities are computed once. */
+ * nb_adjoint_step_dev).  The pair quantities are computed once.  vel and
+ * pos_next must not share memory with pos (equal rows are refused); they may
+ * be rows of lam_x_next / lam_v_next, as lam_x / lam_v of pos above. */
 int nb_fwd_adjoint_step_dev(const nb_params *p, const nb_vec3 *pos,
                             const nb_vec3 *vel, const nb_vec3 *pos_next,
                             const nb_vec3 *lam_x_next,
