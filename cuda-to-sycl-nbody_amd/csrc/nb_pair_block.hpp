@@ -197,8 +197,11 @@ namespace nb {
 #define NB_LIST8(M, o) NB_LIST4(M, o), M(4, o), M(5, o), M(6, o), M(7, o)
 #define NB_IN3(n, k, v, o)                                                     \
   [n##x##k] "v"(v[o]), [n##y##k] "v"(v[o + 1]), [n##z##k] "v"(v[o + 2])
+// early-clobber: the first targets' sums are written before the last targets'
+// inputs are read, so a sum must not share the register of an input whose value
+// it starts from
 #define NB_IO3(n, k, v, o)                                                     \
-  [n##x##k] "+v"(v[o]), [n##y##k] "+v"(v[o + 1]), [n##z##k] "+v"(v[o + 2])
+  [n##x##k] "+&v"(v[o]), [n##y##k] "+&v"(v[o + 1]), [n##z##k] "+&v"(v[o + 2])
 #define NB_OUT3(n, k, v, o)                                                    \
   [n##x##k] "=&v"(v[o]), [n##y##k] "=&v"(v[o + 1]), [n##z##k] "=&v"(v[o + 2])
 #define NB_T_POS(k, o) NB_IN3(t, k, t[o + k], 0)
