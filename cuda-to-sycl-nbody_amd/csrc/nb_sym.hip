@@ -53,6 +53,7 @@
 
 #include "nb_pair_block.hpp"
 #include "nb_pairs.hpp"
+#include "nb_small.hpp"
 
 #include <vector>
 
@@ -119,7 +120,8 @@ struct SymArgs {
 // Finalize arithmetic of the plain rules: row partials are added, the
 // negated reaction partials subtracted, in the order the caller visits them.
 // fetch reads one partial ([ACC] floats, stride apart); add_v / sub_v fold it
-// into the running sums.
+// into the running sums.  merge / unmerge add and subtract running sums inside
+// a work item, where Kahan sums keep both sides' compensation.
 template <int ACC>
 struct PlainPartials {
   static __device__ __forceinline__ void fetch(float (&v)[ACC], const float *p,
@@ -136,6 +138,14 @@ struct PlainPartials {
                                                const float (&v)[ACC]) {
 #pragma unroll
     for (int e = 0; e < ACC; ++e) f[e] = f[e] - v[e];
+  }
+  static __device__ __forceinline__ void merge(float (&f)[ACC],
+                                               const float (&v)[ACC]) {
+    add_v(f, v);
+  }
+  static __device__ __forceinline__ void unmerge(float (&f)[ACC],
+                                                 const float (&v)[ACC]) {
+    sub_v(f, v);
   }
 };
 
@@ -264,6 +274,18 @@ struct KahanForceRule {
                                                const float (&v)[ACC]) {
 #pragma unroll
     for (int e = 0; e < 3; ++e) kahan_value(f, e, v[3 + e] - v[e]);
+  }
+  // The waves' sums may cancel: rounding one to v - c first would leave an
+  // error of the waves' size in the item's sum.
+  static __device__ __forceinline__ void merge(float (&f)[ACC],
+                                               const float (&v)[ACC]) {
+#pragma unroll
+    for (int e = 0; e < 3; ++e) meet(f[e], f[3 + e], v[e], v[3 + e]);
+  }
+  static __device__ __forceinline__ void unmerge(float (&f)[ACC],
+                                                 const float (&v)[ACC]) {
+#pragma unroll
+    for (int e = 0; e < 3; ++e) meet(f[e], f[3 + e], -v[e], -v[3 + e]);
   }
 
   using Own = Particle;
@@ -680,7 +702,7 @@ __device__ __forceinline__ void meet_sources(float (&sum)[U][R::ACC],
         for (int p = 1; p < S::PARTS; ++p) {
           float v[R::ACC];
           R::fetch(v, react + (w + p) * R::ACC * 64 + lane, 64);
-          R::add_v(f, v);
+          R::merge(f, v);
         }
         float *sp = sp_at(g) + set * 64 + lane;
 #pragma unroll
@@ -719,7 +741,7 @@ __device__ __forceinline__ void add_waves(float (&sum)[U][R::ACC], float *lds,
       if (k >= k0 && k < k1) {
         float v[R::ACC];
         R::fetch(v, p + k * 64, RT);
-        R::add_v(sum[k], v);
+        R::merge(sum[k], v);
         __builtin_amdgcn_sched_barrier(0);
       }
   };
@@ -743,12 +765,12 @@ __device__ __forceinline__ void add_waves(float (&sum)[U][R::ACC], float *lds,
       if (held) {
         float v[R::ACC];
         R::fetch(v, held + k * 64 + lane, stride);
-        R::sub_v(sum[k], v);
+        R::unmerge(sum[k], v);
       }
       if constexpr (ADD) {
         float v[R::ACC];
         R::fetch(v, p, stride);
-        R::add_v(v, sum[k]);
+        R::merge(v, sum[k]);
 #pragma unroll
         for (int e = 0; e < R::ACC; ++e) p[e * stride] = v[e];
       } else {
