@@ -5,6 +5,7 @@
 // instead, src/simulator.cuh:22-31).
 
 #include <algorithm>
+#include <atomic>
 #include <cfloat>
 #include <chrono>
 #include <climits>
@@ -62,6 +63,18 @@ namespace {
 // waits for the stream (every earlier use of the buffer was on it), then
 // frees.  Entries are never destroyed; nb_scratch_release frees their
 // buffers.
+//
+// A buffer that cannot grow (its stream is being captured) has to serve what a
+// captured program calls besides the step that sized it: another rule's step
+// on the same particles, a smaller one, the diagnostics.  So a buffer has at
+// least kScratchFloor bytes (Kahan steps up to 12287 particles take 18 MB, the
+// diagnostics up to 6 MB), one-launch steps, which need none, still see to it
+// that there is one, and a larger buffer gets as much again, up to
+// kScratchSpare more (the fused adjoint of a size takes twice the plain step's
+// partials; a smaller size may run a shape with more of them).
+constexpr size_t kScratchFloor = (size_t)32 << 20;
+constexpr size_t kScratchSpare = (size_t)512 << 20;
+
 struct ScratchEntry {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -71,6 +84,7 @@ struct ScratchEntry {
 };
 std::mutex g_scratch_mu; // guards g_scratch (the list, not the entries)
 std::vector<std::unique_ptr<ScratchEntry>> g_scratch;
+std::atomic<unsigned> g_scratch_releases{0};
 
 ScratchEntry *scratch_entry(int dev, hipStream_t stream) {
   std::lock_guard<std::mutex> lock(g_scratch_mu);
@@ -109,13 +123,57 @@ int acquire_scratch(size_t bytes, hipStream_t stream, ScratchLease &lease) {
       e->bytes = 0;
     }
     void *p = nullptr;
-    if ((st = hip_check(hipMalloc(&p, bytes), "scratch hipMalloc"))) return st;
+    size_t size = std::max(kScratchFloor, bytes + std::min(bytes, kScratchSpare));
+    if (hipMalloc(&p, size) != hipSuccess) { // no room to spare: the need alone
+      (void)hipGetLastError();
+      size = bytes;
+      if ((st = hip_check(hipMalloc(&p, size), "scratch hipMalloc"))) return st;
+    }
     e->ptr = static_cast<float *>(p);
-    e->bytes = bytes;
+    e->bytes = size;
   }
   lease.ptr_ = e->ptr;
   lease.lock_ = std::move(lock);
   return NB_OK;
+}
+
+void reserve_scratch(hipStream_t stream) {
+  // The look-up takes 80 ns of a 3 us call, so a thread keeps the last stream
+  // it found a buffer for, until buffers are released; with one device only,
+  // where the stream alone names the entry.
+  static const bool one_device = [] {
+    int count = 0;
+    return hipGetDeviceCount(&count) == hipSuccess && count == 1;
+  }();
+  thread_local hipStream_t seen = nullptr;
+  thread_local unsigned seen_at = ~0u; // releases when it was found
+  const unsigned releases = g_scratch_releases.load(std::memory_order_relaxed);
+  if (one_device && seen == stream && seen_at == releases) return;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return;
+  ScratchEntry *e = scratch_entry(dev, stream);
+  std::unique_lock<std::mutex> lock(e->mu, std::try_to_lock);
+  if (!lock.owns_lock()) return; // a lease holds it: it has a buffer
+  if (e->ptr) {
+    seen = stream;
+    seen_at = releases;
+    return;
+  }
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) == hipSuccess &&
+      cap == hipStreamCaptureStatusNone) {
+    // relaxed: the call must not disturb a capture of another stream
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {
+      void *p = nullptr;
+      if (hipMalloc(&p, kScratchFloor) == hipSuccess) {
+        e->ptr = static_cast<float *>(p);
+        e->bytes = kScratchFloor;
+      }
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+  }
+  (void)hipGetLastError(); // the step itself needs none
 }
 
 } // namespace nb
@@ -133,6 +191,7 @@ extern "C" int nb_scratch_release(void) {
   for (auto &e : g_scratch)
     if (e->device == dev) held.emplace_back(e->mu);
   if ((st = hip_check(hipDeviceSynchronize(), "device synchronize"))) return st;
+  ++g_scratch_releases;
   for (auto &e : g_scratch) {
     if (e->device != dev) continue;
     if (e->ptr) (void)hipFree(e->ptr);
@@ -675,6 +734,7 @@ int nb_forward_step_dev(const nb_params *p, const float *px, const float *py,
   if (st || n == 0) return st;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   ScratchLease lease; // held until the launches are enqueued
+  if (forward_one_launch(cfg)) reserve_scratch(s);
   if ((st = acquire_scratch(forward_scratch_bytes(cfg, n, mode), s, lease)))
     return st;
   return launch_forward(consts_of(p), mode, cfg, px, py, pz, vx, vy, vz, nx,

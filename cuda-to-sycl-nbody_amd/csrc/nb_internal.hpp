@@ -198,6 +198,9 @@ class ScratchLease {
 // `bytes` (0: none) of scratch for launches on `stream`.  Refuses to grow a
 // buffer while the stream is being captured into a graph.
 int acquire_scratch(size_t bytes, hipStream_t stream, ScratchLease &lease);
+// Gives `stream` a first buffer, for later calls under capture, if it has none
+// and is not being captured.  Never fails.
+void reserve_scratch(hipStream_t stream);
 
 // SoA -> AoS vec4 pack on the device (out: 4 n floats, 16 B aligned).
 // Copies six device arrays of n floats to dst + c * stride (c = 0..5), a

@@ -75,6 +75,7 @@ int adjoint_common(const nb_params *p, const nb_vec3 *pos, const nb_vec3 *vel,
   }
   const hipStream_t s = static_cast<hipStream_t>(stream);
   ScratchLease scratch; // held until the launches are enqueued
+  if (adjoint_one_launch(cfg)) reserve_scratch(s);
   if ((st = acquire_scratch(adjoint_scratch_bytes(cfg, n), s, scratch))) return st;
   const float *P[3] = {pos->x, pos->y, pos->z};
   const float *LXN[3] = {lxn->x, lxn->y, lxn->z};

@@ -255,7 +255,10 @@ int nb_forward_config_scheme(int cfg);
  * never share it, and a call that needs more grows it (after waiting for the
  * stream).  A call that would grow it while its stream is being captured
  * into a graph fails with NB_ERR_UNSUPPORTED; make the call once before
- * capturing.
+ * capturing.  A buffer has at least 32 MiB (one-launch steps, which need none,
+ * allocate it too) and else twice what the call needs, with at most 512 MiB to
+ * spare, so that a captured step of another rule or fewer particles, or a
+ * captured diagnostic, mostly finds enough.
  *   nb_scratch_release  waits for all work on the current device, then frees
  *                       every such buffer of the device (they are allocated
  *                       again on demand);
