@@ -784,10 +784,11 @@ int nb_forward_step_noalloc_dev(const nb_params *p, const float *px,
                              &cfg, &mode);
   if (st || n == 0) return st;
   const size_t bytes = forward_scratch_bytes(cfg, n, mode);
-  if (bytes > kStaticScratchBytes)
+  const size_t counted = forward_noalloc_bytes(cfg, n, mode);
+  if (std::max(bytes, counted) > kStaticScratchBytes)
     return set_error(NB_ERR_UNSUPPORTED,
-                     "the launch shape needs " + std::to_string(bytes) +
-                         " bytes of scratch at n = " + std::to_string(n) +
+                     "the launch shape counts " + std::to_string(counted) +
+                         " bytes of partial sums at n = " + std::to_string(n) +
                          ", more than the 64 MiB static buffer of the "
                          "allocation-free step: use nb_forward_step_dev or a "
                          "shape with fewer partial sums");

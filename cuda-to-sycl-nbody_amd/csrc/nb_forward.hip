@@ -368,6 +368,15 @@ size_t forward_scratch_bytes(int cfg, size_t n, int mode) {
   return c.split > 1 ? sizeof(float) * 3 * (size_t)c.split * n : 0;
 }
 
+size_t forward_noalloc_bytes(int cfg, size_t n, int mode) {
+  const FwdConfig &c = kConfigs[cfg];
+  if (c.scheme != SCHEME_SYMMETRIC_TILES || n > kSymTileMaxParticles)
+    return forward_scratch_bytes(cfg, n, mode);
+  const bool kahan = mode == MODE_KAHAN || mode == MODE_KAHAN_SKIP;
+  const size_t P = c.tile, T = (n + P - 1) / P;
+  return sizeof(float) * (kahan ? 6 : 3) * T * (T + 1) * P * c.split;
+}
+
 int launch_forward(const StepConsts &c, int mode, int cfg, const float *px,
                    const float *py, const float *pz, float *vx, float *vy,
                    float *vz, float *nx, float *ny, float *nz, int n,

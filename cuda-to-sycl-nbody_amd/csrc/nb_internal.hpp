@@ -174,10 +174,14 @@ int launch_forward(const StepConsts &c, int mode, int cfg, const float *px,
                    float *vz, float *nx, float *ny, float *nz, int n,
                    float *scratch, hipStream_t stream);
 
-// Bytes of scratch launch_forward needs for (cfg, n, pair mode).
 // Kernel launches of one step (a banded step takes more).
 int forward_launches(int cfg);
+// Bytes of scratch launch_forward needs for (cfg, n, pair mode).
 size_t forward_scratch_bytes(int cfg, size_t n, int mode);
+// The bytes that decide whether the allocation-free step takes a call: its
+// limits are part of the interface and stay where they are stated (tile pairs:
+// two partials per pair of tiles and item), whatever the kernels use of it.
+size_t forward_noalloc_bytes(int cfg, size_t n, int mode);
 
 // Scratch owned by the library: one buffer per (device, stream), grown on
 // demand and freed by nb_scratch_release.  A lease holds the buffer's lock:

@@ -1375,15 +1375,10 @@ size_t sym_scratch_bytes(int unroll, int chunk, size_t n, int acc,
                          bool tiles, bool bandable) {
   if (tiles) {
     if (n == 0 || n > sym_max_particles(unroll, tiles, chunk, acc)) return 0;
-    // the limits of the callers' buffers are stated in tile pairs: a row and a
-    // reaction partial per pair and item; the row form needs no more from the
-    // second tile on
-    const long long P = 64LL * unroll;
-    const long long T = ((long long)n + P - 1) / P;
+    // ts (ts + 1) / 2 row partials and ts (ts - 1) / 2 reaction partials
     const long long st = 64LL * tile_targets(unroll, chunk, n);
     const long long ts = ((long long)n + st - 1) / st;
-    return sizeof(float) * acc *
-           (size_t)std::max(T * (T + 1) * P * std::max(chunk, 1), ts * ts * st);
+    return sizeof(float) * acc * (size_t)(ts * ts * st);
   }
   if (bandable && sym_banded(unroll, tiles, chunk, acc, n)) {
     const BandPlan bp = band_plan(n, unroll, chunk);

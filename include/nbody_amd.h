@@ -201,7 +201,9 @@ int nb_forward_step_dev(const nb_params *p, const float *px, const float *py,
  * 12800 and the 25600 of its CPU configuration among them; Kahan sums up to
  * n = 18816).  Nothing in it needs clearing between calls: every partial
  * sum is written before it is read.  A shape whose partial sums
- * exceed it is refused with NB_ERR_UNSUPPORTED.  Every call on one GPU uses
+ * exceed it is refused with NB_ERR_UNSUPPORTED; the tile-pair shapes count two
+ * partials per pair of tiles and item, about twice what they write from 9728
+ * particles on.  Every call on one GPU uses
  * that GPU's buffer: calls that overlap on one GPU (different streams or
  * host threads) race and must be ordered by the caller. */
 int nb_forward_step_noalloc_dev(const nb_params *p, const float *px,
