@@ -4,7 +4,10 @@
 // (v_mov_b32_dpp wave_rol:1) and the forward pair term of the symmetric
 // kernels (3 sub, 3 fma, 2 mul, v_rsq_f32, 6 fma), each as one long
 // dependent chain per lane (latency) and as several independent chains
-// (throughput), at 1..4 waves per SIMD.
+// (throughput), at 1..4 waves per SIMD.  Loops with registers fixed in assembly
+// show what the pair term's block (csrc/nb_pair_block.hpp) is written for: the
+// register banks of a three-operand FMA, and what a v_rsq_f32 does to the FMAs
+// after it with and without a non-VALU instruction beside it.
 //
 // Every kernel works in registers only and writes one float per thread
 // (keeps the chains alive) and, from lane 0 of each wave, the wave's shader
@@ -64,12 +67,35 @@ enum Op : int {
   OP_ADD_S = 10,   // v_add_f32_e32 with an SGPR first operand
   OP_FMA_VVV = 11, // v_fma_f32 (VOP3), VGPR operands only
   OP_FMAC_SQ = 12, // v_fmac_f32_e32 d, r, r (two distinct VGPRs read)
+  // fixed registers (one chain = one block of instructions):
+  OP_BANK_MIX = 13,  // 14 v_fmac: odd sums, even factors
+  OP_BANK_EVEN = 14, // 14 v_fmac, sums and factors even
+  OP_RSQ_BARE = 15,  // v_rsq_f32 + the 14 of OP_BANK_MIX
+  OP_RSQ_NOP = 16,   // the same, an s_nop after the v_rsq
+  OP_RSQ_PRIO = 17,  // the same, s_setprio 1 / 0 around the v_rsq
 };
+
+// Registers v32 .. v63 (never initialised: only the issue is timed).
+#define FMAC(d) "v_fmac_f32 v" #d ", v60, v62\n\t"
+#define FMAC14_ODD                                                            \
+  FMAC(33) FMAC(35) FMAC(37) FMAC(39) FMAC(41) FMAC(43) FMAC(45) FMAC(47)      \
+  FMAC(49) FMAC(51) FMAC(53) FMAC(55) FMAC(57) FMAC(59)
+#define FMAC14_EVEN                                                           \
+  FMAC(32) FMAC(34) FMAC(36) FMAC(38) FMAC(40) FMAC(42) FMAC(44) FMAC(46)      \
+  FMAC(48) FMAC(50) FMAC(52) FMAC(54) FMAC(56) FMAC(58)
+#define RSQ "v_rsq_f32 v61, v63\n\t"
+#define FIXED_REGISTERS                                                       \
+  "v32", "v33", "v34", "v35", "v36", "v37", "v38", "v39", "v40", "v41", "v42", \
+      "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52",    \
+      "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62",    \
+      "v63"
 
 // Instructions one chain step issues (the loop counter adds a few SALU/VALU
 // per trip, not counted: < 1 % at kUnroll x CHAINS >= 16).  The mixed cases
 // count their extra instruction per 2 steps in steps_insts below.
 constexpr int insts_per_step(int op) {
+  if (op >= OP_RSQ_BARE) return 15; // v_rsq_f32 + 14 v_fmac
+  if (op >= OP_BANK_MIX) return 14;
   return op == OP_PAIR ? 16 : 1; // pair: 14 VALU + v_rsq_f32 + the link
 }
 
@@ -131,6 +157,19 @@ __global__ __launch_bounds__(kBlock) void chain_kernel(Out o, int iters,
             if constexpr (OP == OP_MIX_RSQ) v = __builtin_amdgcn_rsqf(v);
             else v = wave_rol1(v);
           }
+        } else if constexpr (OP == OP_BANK_MIX) {
+          asm volatile(FMAC14_ODD : : : FIXED_REGISTERS);
+        } else if constexpr (OP == OP_BANK_EVEN) {
+          asm volatile(FMAC14_EVEN : : : FIXED_REGISTERS);
+        } else if constexpr (OP == OP_RSQ_BARE) {
+          asm volatile(RSQ FMAC14_ODD : : : FIXED_REGISTERS);
+        } else if constexpr (OP == OP_RSQ_NOP) {
+          asm volatile(RSQ "s_nop 0\n\t" FMAC14_ODD : : : FIXED_REGISTERS);
+        } else if constexpr (OP == OP_RSQ_PRIO) {
+          asm volatile("s_setprio 1\n\t" RSQ "s_setprio 0\n\t" FMAC14_ODD
+                       :
+                       :
+                       : FIXED_REGISTERS);
         } else {
           // forward pair term: source a[c] (+ offsets) against target t[c];
           // target sums b[c], reaction sums s[c]; the next step's source
@@ -201,6 +240,11 @@ int main(int argc, char **argv) {
       make<OP_MIX_RSQ, 7>("fmac14+rsq"), make<OP_MIX_DPP, 8>("fmac16+dpp"),
       make<OP_ADD_S, 8>("add_sgpr x8"), make<OP_FMA_VVV, 8>("fma_vop3 x8"),
       make<OP_FMAC_SQ, 8>("fmac_sq x8"),
+      make<OP_BANK_MIX, 1>("fmac mixed banks"),
+      make<OP_BANK_EVEN, 1>("fmac one bank"),
+      make<OP_RSQ_BARE, 1>("rsq + 14 fmac"),
+      make<OP_RSQ_NOP, 1>("rsq, s_nop + 14"),
+      make<OP_RSQ_PRIO, 1>("rsq, setprio + 14"),
   };
   const int wps_list[] = {1, 2, 3, 4}; // waves per SIMD
   const int max_groups = cus * 4;
@@ -222,7 +266,9 @@ int main(int argc, char **argv) {
       const int groups = cus * wps; // one 4-wave group per CU per wave/SIMD
       const int waves = groups * (kBlock / 64);
       // pair cases carry 15 instructions per step: fewer trips
-      const int it = c.op == OP_PAIR ? std::max(1, iters / 8) : iters;
+      const int it = c.op == OP_PAIR || c.op >= OP_BANK_MIX
+                         ? std::max(1, iters / 8)
+                         : iters;
       Out o{val, cyc, rt};
       void *args[] = {&o, const_cast<int *>(&it), nullptr};
       float x = 0.999f;
@@ -254,7 +300,7 @@ int main(int argc, char **argv) {
       // the same from the event time, at the measured clock
       const double ev_per_cu =
           insts * waves / (ms * 1e-3 * ghz * 1e9) / cus;
-      std::printf("%-9s waves/SIMD %d: cyc/inst %6.2f  simd_cpi %6.2f  "
+      std::printf("%-17s waves/SIMD %d: cyc/inst %6.2f  simd_cpi %6.2f  "
                   "per_cu_clk %5.3f  (event: %5.3f)  %.3f GHz  %.3f ms\n",
                   c.name, wps, cpi, simd_cpi, per_cu, ev_per_cu, ghz, ms);
       char buf[320];
