@@ -430,24 +430,23 @@ const FwdConfig &adjoint_config(int cfg) { return kAdjConfigs[cfg]; }
 
 int adjoint_default_config(size_t n, bool skip) {
   // Measured on MI355X (disk ICs), adjoint / fused us (device time).  One
-  // launch, and tile pairs, 2 per lane: n = 32 2.9 / 3.4 and 6.8 / 7.8
-  // (target-sharded 256 x 1 split 2 5.4 / 5.7), 1000 4.0 / 4.9 and 8.7 / 10.2
-  // (58 / 67), 2000 6.9 / 8.2 and 9.2 / 10.9, 2500 11.7 / 13.4 and 9.7 / 11.5,
-  // 4000 17.1 / 19.2 and 15.1 / 18.4.  Tile pairs: 4097 15.1 / 19.1 (63 / 72),
-  // 12800 53.5 / 70.6, 24000 162 / 215 (super-tiles of 512, 1 per item 176 /
-  // 229), 30720 264.1 / 350.4 (274.5 / 359.1), 34000 321.8 / 428.6 (313.3 /
-  // 407.4).
-  // Super-tiles of 512, 1 / 2 per item: 65536 1041 / 1369 vs 1052 / 1411 (tile
-  // pairs 1099 / 1490), 100000 2371 / 3160 vs 2360 / 3124, 262144 16154 / 21434 vs 15812 / 21092 (super-tiles of 1024:
-  // 16461 / 22713 on a card where 2 per item took 16509 / 21775).  Best
-  // target-sharded at 262144 31.5 / 39.0 ms.  Past 2^18 four super-tiles per
-  // item and bands of source super-tiles.
+  // launch, and tile pairs: n = 32 2.8 / 3.4 and 6.6 / 7.7 (target-sharded 256 x
+  // 1 split 2 5.2 / 5.8), 1000 4.1 / 4.9 and 8.7 / 10.2 (58 / 67), 2000 6.6 /
+  // 7.9 and 9.0 / 10.7, 2500 11.2 / 13.1 and 9.3 / 11.0, 4000 16.1 / 18.6 and
+  // 13.9 / 17.1.  Tile pairs: 4097 15.3 / 19.3 (target-sharded 63 / 72), 12800
+  // 52.4 / 69.2, 24000 163 / 216 (super-tiles of 512, 1 per item 197 / 228),
+  // 30720 258 / 341 (269 / 349), 34000 315 / 419 (307 / 396).
+  // Super-tiles of 512, 1 / 2 per item: 65536 1061 / 1386 vs 1090 / 1421 (tile
+  // pairs 1113 / 1506), 100000 2416 / 3192 vs 2415 / 3167, 262144 16725 / 22162
+  // vs 16551 / 21894 (super-tiles of 1024 16441 / 21557).  Best target-sharded at
+  // 262144 30.7 / 40.0 ms.  Past 2^18 four super-tiles per item and bands of
+  // source super-tiles.
   if (n <= kSymBandedMaxParticles && n > kSymSmallMaxParticles)
     return 22; // super-tile pairs, 2 per lane, 4 per item, in bands
   if (n <= kSymMaxParticles) { // skip or not: self pairs masked in-kernel
     if (n >= 98304) return 20; // super-tile pairs, 2 per lane, 2 per item
     if (n >= 32768) return 19; // super-tile pairs, 2 per lane, 1 per item
-    if (n > 2048) return 18;   // tile pairs, 2 per lane
+    if (n > 2048) return 18;   // tile pairs
     return 23;                 // one launch
   }
   return 8; // 256 x 1, split 2

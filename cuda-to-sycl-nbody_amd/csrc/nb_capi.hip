@@ -452,7 +452,8 @@ int nb_sim_create(const nb_params *p, const float *px, const float *py,
 
 // Launches of a frame up to which they are issued one by one: a graph costs
 // some 16 us before its first kernel, direct launches fall behind from the
-// sixth on.  Frame, graph / direct, us: n = 500 2 steps 36.7 / 19.3, 5 38.0 /
+// sixth on (at n = 500 the sixth adds 20 us to the frame and 6 to its device
+// time; why is not known, so the line is where the measurements put it).  Frame, graph / direct, us: n = 500 2 steps 36.7 / 19.3, 5 38.0 /
 // 29.5, 6 40 / 51, 8 45 / 56 (one launch a step); 4097 2 steps 47.5 / 38.4, 3
 // 58.4 / 59, 8 120 / 123; 20000 2 steps 189 / 178 (two launches a step).
 static constexpr long long kDirectLaunches = 5;

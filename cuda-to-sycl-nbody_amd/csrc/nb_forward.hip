@@ -242,10 +242,11 @@ const ShapeEntry kShapes[] = {
 
 // Compiled launch shapes: {block, unroll, tile, split[, scheme]}.  Index 0
 // must stay the unsplit 256 x 1 shape (a valid choice for every n).  The
-// symmetric shapes (nb_sym.hip) are {256, particles per lane, super-tile,
-// super-tiles per work item}, where 256 x particles per lane is the super-tile:
-// the workgroups have 256 threads, 512 with 8 per lane and for tile pairs of 2
-// per lane below 3328 particles.
+// symmetric shapes (nb_sym.hip) are {256, u, super-tile, super-tiles per work
+// item} with super-tiles of 256 u: a wave holds rows of 512, 8 per lane, in
+// workgroups of 256 threads (512 with u = 8).  Tile pairs {256, 2, 128, 1} run
+// rows of 128 below 9728 particles (512 threads below 3328) and of 256, 4 per
+// lane, from there, {256, 4, 256, 1} always the latter.
 const FwdConfig kConfigs[] = {
     {256, 1, 1024, 1}, {256, 1, 1024, 2}, {256, 1, 1024, 4},
     {256, 1, 1024, 8}, {256, 2, 1024, 1}, {256, 2, 1024, 2},
@@ -264,7 +265,7 @@ const FwdConfig kConfigs[] = {
     {256, 2, 128, 1, SCHEME_SYMMETRIC_TILES},
     {256, 2, 512, 1, SCHEME_SYMMETRIC}, {256, 2, 512, 2, SCHEME_SYMMETRIC},
     {256, 2, 512, 4, SCHEME_SYMMETRIC},
-    {256, 2, 128, 2, SCHEME_SYMMETRIC_TILES}, // two items per tile pair
+    {256, 2, 128, 2, SCHEME_SYMMETRIC_TILES}, // tile pairs, rows of 128 at every n
     {kSmallBlock, 1, 1024, 1},                // one launch (fwd_small_kernel)
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
@@ -288,39 +289,38 @@ int forward_default_config(size_t n, int mode) {
   if (mode == MODE_PLAIN_SKIP) mode = MODE_PLAIN;
   if (mode == MODE_KAHAN_SKIP) mode = MODE_KAHAN;
   // Measured on MI355X (disk ICs), us per step (device time), best others in
-  // brackets.  Tile pairs, 2 per lane: n = 4097 13.5 (target-sharded 40), 12000
-  // 38.2 (super-tiles of 512, 1 per item 49.8), 28000 141.1 (150.5), 32768
-  // 189.4 (191.6), 36000 227.6 (222.0), 49000 405.5 (387.5).  Super-tiles win
-  // from about 34000; the line stays at 49152 because the tile pairs' partials
-  // (64 to 217 MiB at 26752 to 49151) are what makes the allocation-free step
-  // refuse those sizes, and super-tiles (54 MiB) would have it accept them.
-  // Super-tiles of 512, 1 per item: 50021 379 (tile pairs 412, 1024 412), 52000
-  // 426.2 (453.8), 65536 652 (677 with 1024), 100000 1465 (1468 with 2 per
-  // item, 1470 with 1024).  Of 1024:
-  // 131072 2489 (2496 with 512, 2605 with 2048), 200000 5734 (5757, 5789),
-  // 262144 9786 (2048: 9868, with a quarter of the scratch's growth: the
-  // choice from there).  Past 2^19 two super-tiles of 2048 per item need 25 %
-  // less scratch; past 2^20 four per item keep the partials at 16 GB for 2^21
-  // particles, and past 2^21 the step runs in bands of source super-tiles with
-  // at most 8 GB of partials each (the 4-per-lane shape with 4 per item is
-  // banded past 2^20).
+  // brackets.  Tile pairs: n = 4097 11.7 (target-sharded 40), 12000 35.4
+  // (super-tiles of 512, 1 per item 49.0), 28000 137 (148), 32768 184 (188),
+  // 36000 222 (215), 49000 397 (380).  Super-tiles win from about 34000; the
+  // line is at 49152 because the allocation-free step's limits are counted for
+  // the default shape: a super-tile default would have it accept sizes that it
+  // refuses (26625 to 49151).  Super-tiles of 512, 1 per item: 50021 383 (tile
+  // pairs 416, 1024 417), 52000 419 (448), 65536 647 (674 with 1024), 100000
+  // 1471 (1468 with 2 per item, 1472 with 1024).  Of 1024: 131072 2488 (2509
+  // with 512, 2605 with 2048), 200000 5849 (6001, 5895), 262144 10035 (2048:
+  // 10150, with a quarter of the scratch's growth: the choice from there).  Past
+  // 2^19 two super-tiles of 2048 per item need 25 % less scratch; past 2^20 four
+  // per item keep the partials at 16 GB for 2^21 particles, and past 2^21 the
+  // step runs in bands of source super-tiles with at most 8 GB of partials each
+  // (the 4-per-lane shape with 4 per item is banded past 2^20).
+  // Shapes 33 and 37 run the same kernels below 9728 particles; 37 stays the
+  // name of the default below 6656.
   if (mode == MODE_PLAIN && n <= kSymBandedMaxParticles) {
     if (n > kSymMaxParticles) return 24; // 8 per lane, 4 per item (banded past 2^21)
     if (n > ((size_t)1 << 19)) return 23;  // symmetric, 8 per lane, 2 per item
     if (n >= ((size_t)1 << 18)) return 22; // symmetric, 8 per lane, 1 per item
     if (n >= ((size_t)1 << 17)) return 25; // symmetric, 4 per lane, 1 per item
     if (n >= 49152) return 34;             // symmetric, 2 per lane, 1 per item
-    if (n >= 6656) return 33;              // symmetric tile pairs, 2 per lane
-    if (n >= 4096) return 37;              // the same, two items per tile pair
+    if (n >= 6656) return 33;              // symmetric tile pairs
+    if (n >= 4096) return 37;              // the same
   }
-  // Kahan, us per step: tile pairs, 2 per lane: n = 4097 20 (best split
-  // target-sharded 56), 5000 22.2 (one launch 22.6), 12000 67 (123), 32000 324 (572);
-  // super-tiles of 512, 1 per item, and tile pairs: 32768 362.6 and 353.8,
-  // 36000 421.9 and 427.0, 40960 517.8 and 540.3, 49000 738.2 and 765.4 (below
-  // 40960 the same reason as above).  1 / 2 per item: 100000 2830 / 2809,
-  // 262144 19295 / 18999 (target-sharded 28751).  Above 2^18 four super-tiles
-  // per item run in bands of source super-tiles (16 GB of (sum, compensation)
-  // partials per band).
+  // Kahan, us per step: tile pairs: n = 4097 18.0 (best split target-sharded
+  // 56), 5000 21.1 (one launch 33.5), 12000 64 (123), 32000 327 (575);
+  // super-tiles of 512, 1 per item, and tile pairs: 32768 355 and 346, 36000
+  // 416 and 418, 40960 506 and 529, 49000 724 and 750 (below 40960 the same
+  // reason as above).  1 / 2 per item: 100000 2867 / 2862, 262144 19921 / 19648
+  // (target-sharded 28993).  Above 2^18 four super-tiles per item run in bands
+  // of source super-tiles (16 GB of (sum, compensation) partials per band).
   if (mode == MODE_KAHAN) {
     if (n > ((size_t)1 << 18) && n <= kSymBandedMaxParticles)
       return 36;               // symmetric, 2 per lane, 4 per item, banded
@@ -329,12 +329,12 @@ int forward_default_config(size_t n, int mode) {
     if (n >= 40960 && n < ((size_t)1 << 17))
       return 34;               // symmetric, 2 per lane, 1 per item
     if (n >= 4096 && n < 40960)
-      return 33;               // symmetric tile pairs, 2 per lane
+      return 33;               // symmetric tile pairs
   }
   // One launch, plain / Kahan us (device time; split target-sharded plain,
-  // then tile pairs plain / Kahan): n = 64 2.9 / 3.5 (10.5, 6.4 / 8.0), 1000
-  // 3.4 / 4.2 (23.8, 8.5 / 10.6), 2000 4.6 / 6.7 (24.0, 9.0 / 11.2), 4000
-  // 8.9 / 15.3 (24.8, 11.9 / 17.6); tile pairs from 4096.
+  // then tile pairs plain / Kahan): n = 64 2.9 / 3.3 (10.8, 5.8 / 7.5), 1000
+  // 3.3 / 4.2 (24.0, 7.4 / 9.4), 2000 4.6 / 6.7 (24.0, 7.8 / 9.9), 4000
+  // 8.9 / 15.4 (24.9, 10.9 / 16.8); tile pairs from 4096.
   if (n < 4096) return 38;
   // Target-sharded, Gint/s: n = 4096: 128 x 1 split 8 629 (256 x 1 split 8
   // 480); 8192: 256 x 1 split 8 1746 (split 16 1629); 16384 .. 32768:

@@ -46,15 +46,16 @@ enum PairMode : int {
 enum FwdScheme : int {
   SCHEME_TARGETS = 0,   // each thread sums all sources for its targets
   SCHEME_SYMMETRIC = 1, // each pair term evaluated once, applied to both;
-                        // work item = super-tile pair (4 waves)
-  SCHEME_SYMMETRIC_TILES = 2, // the same, work item = tile pair (one wave)
+                        // work item = a row chunk of super-tile pairs
+  SCHEME_SYMMETRIC_TILES = 2, // the same with small super-tiles, one pair an item
 };
 
-// One compiled launch shape of the forward kernel.  For SCHEME_SYMMETRIC
-// (nb_sym.hip): block = 256 (4 waves), unroll = particles per lane,
-// tile = super-tile length (4 * 64 * unroll), split = super-tiles per work
-// item (row chunk).  For SCHEME_SYMMETRIC_TILES: tile = tile length
-// (64 * unroll), split = 1.
+// One compiled launch shape of the forward kernel.  For the symmetric schemes
+// (nb_sym.hip) the fields name the shape; the kernels' own workgroups and
+// targets per lane are chosen from them and n (find_shape).  SCHEME_SYMMETRIC:
+// unroll and tile = super-tile length (256 * unroll), split = super-tiles per
+// work item.  SCHEME_SYMMETRIC_TILES: unroll and tile = 64 * unroll; split 2:
+// rows of 128 at every n.
 struct FwdConfig {
   int block;  // threads per workgroup
   int unroll; // target particles per thread

@@ -4,16 +4,16 @@
 // rounding, same order of every sum: the results are the same bits).
 //
 // Why assembly.  Two waves of a SIMD issue fp32 VALU instructions together,
-// 2 cycles each, under two conditions measured with register-only loops:
+// 2 cycles each, under two conditions (probe/issue_rates.hip, 2 waves):
 //   * the three sources of an FMA must not all be even or all be odd VGPRs
 //     (two banks, two reads each; a register read twice counts twice), and
-//     none may be an SGPR: 4 cycles otherwise.  The compiler's allocation
-//     broke this for 194 of 512 v_fmac and, with eps in an SGPR, for every
-//     first FMA of |r|^2 + eps;
-//   * after a v_rsq_f32 the two waves stay out of step, and every later
-//     instruction takes 4 cycles, until one of them issues a non-VALU
-//     instruction: v_rsq + 14 FMAs take 64 cycles bare, 38 with an s_nop or
-//     an s_setprio beside the v_rsq.
+//     none may be an SGPR: v_fmac 2.2 cycles with mixed registers, 4.2 with all
+//     even, 4.2 with an SGPR.  The compiler's allocation broke this for 194 of
+//     512 v_fmac and, with eps in an SGPR, for every first FMA of |r|^2 + eps;
+//   * after a v_rsq_f32 the two waves stay out of step, and later instructions
+//     take up to 4 cycles, until one of them issues a non-VALU instruction:
+//     v_rsq + 14 FMAs take 51 cycles bare, 39 with an s_nop behind the v_rsq, 41
+//     with an s_setprio on either side.
 // So r and h (see AdjointRule) sit in even temporaries, d, K and t3 in odd
 // ones: every FMA below mixes the two whatever registers the compiler gives
 // the sums.  eps is pinned to an odd register.  Each v_rsq is bracketed by
@@ -23,10 +23,12 @@
 // sums of one are issued behind the v_rsq of the next; v_rsq results are
 // read at least one instruction later (its hazard).
 //
-// Measured (forward, 8 sources x 8 targets per step, sustained): 45.6 SIMD
-// cycles per wave pair term at 3 waves per SIMD against 49.6 for the
-// compiler's loop; from 4 waves on power limits both (44.6 against 47.2).  The
-// kernels' 1 source x 8 targets: 46.9 at 4 waves.
+// Measured, the pair loop alone (forward, 8 sources x 8 targets per step,
+// sustained; time at 2.4 GHz): 45.6 cycles per wave pair term at 3 waves per
+// SIMD against 49.6 for the compiler's loop; at 4 waves 44.6 against 47.2.  The
+// kernels' 1 source x 8 targets: 46.9 at 4 waves.  In the step at N = 262144 the
+// counters give 40.6 clock cycles a term at 1.8 to 2.1 GHz (48.6 at 2.26 GHz
+// before): the cycles are the same in every launch, the clock is what varies.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -1178,12 +1178,12 @@ constexpr SymShape sym_shape() {
           four ? kThirdOfLds - lds : 0};
 }
 
-// Targets per lane of a tile-pair shape: `unroll` particles per lane and
-// tile (tiles of 64 * unroll), `items` work items per tile pair.  With two
-// items, and below kTilePairRows particles, tiles of 2 per lane are taken one
-// at a time (super-tiles of 128, two waves per set of sources: four times the
-// workgroups); from there two at a time (4 targets per lane, half the LDS
-// traffic and partials per pair term).  Both sides, us per step, device time
+// Targets per lane of a tile-pair shape of `unroll` particles per lane (tiles
+// of 64 * unroll).  Below kTilePairRows particles tiles of 2 per lane are taken
+// one at a time (super-tiles of 128, two waves per set of sources: four times
+// the workgroups); from there two at a time (4 targets per lane, half the LDS
+// traffic and partials per pair term).  `items` 2 names the shape that keeps
+// rows of 128 at every size.  Both sides, us per step, device time
 // (forward / Kahan / adjoint / fused): n = 4097 11.8 / 17.7 / 15.1 / 19.1 vs
 // 17.9 / 26.6 / 23.7 / 28.5, 9000 26.8 / 42.8 / 35.5 / 46.7 vs 25.5 / 44.2 /
 // 38.5 / 49.4, 9728 29.9 / 48.6 / 39.9 / 52.8 vs 25.8 / 44.8 / 36.6 / 47.2,
@@ -1345,7 +1345,7 @@ int launch_sym(const SymShape *sh, SymArgs &a, int unroll, int chunk, int n,
     if (chunk > 2)
       return set_error(NB_ERR_UNSUPPORTED,
                        "tile-pair shapes take one or two items per tile pair");
-    chunk = 1; // one super-tile pair per work item
+    chunk = 1; // one super-tile pair per work item, whatever the shape's name
   }
   const int ts = (n + sh->st - 1) / sh->st;
   const long long blocks = items_upto(ts, chunk);

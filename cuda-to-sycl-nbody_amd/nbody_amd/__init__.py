@@ -119,8 +119,10 @@ def forward_config_info(cfg: int) -> dict:
     each thread sums all sources for its targets; "symmetric": each pair term
     evaluated once and applied to both particles, where tile is the
     super-tile length and split the super-tiles per work item;
-    "symmetric_tiles": the same with one tile pair per wave, tile = the tile
-    length)."""
+    "symmetric_tiles": the same with small super-tiles, tile = the tile length,
+    split 2 the shape that keeps rows of 128).  The symmetric fields name the
+    shape; workgroup size and targets per lane of the kernels follow from it
+    and n."""
     lib = load()
     vals = [ctypes.c_int() for _ in range(4)]
     check(lib.nb_forward_config_info(cfg, *[ctypes.byref(v) for v in vals]))

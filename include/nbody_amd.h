@@ -162,10 +162,10 @@ int nb_sim_set_accumulation(nb_sim *s, int mode);
 /* Changes simIterationsPerFrame for later nb_sim_step calls. */
 int nb_sim_set_frame_iterations(nb_sim *s, int iters);
 
-/* Frames of more than five launches (a step takes one launch below 4096
- * particles, two from there; nb_sim_step, nb_sim_advance) are captured once
- * as a hipGraph per (steps, launch shape, accumulation, start buffer) and
- * replayed; enable = 0 launches every step directly (results are the same
+/* Frames of more than five launches (nb_sim_step, nb_sim_advance; with the
+ * default shapes a step takes one launch below 4096 particles, two from there,
+ * more in bands) are captured once as a hipGraph per (steps, launch shape,
+ * accumulation, start buffer) and replayed; enable = 0 launches every step directly (results are the same
  * bits).  No counterpart in the reference, whose stepSim launches each step
  * (src/simulator.cu:59-66).  Default: on. */
 int nb_sim_set_graph(nb_sim *s, int enable);
@@ -214,8 +214,11 @@ int nb_forward_step_noalloc_dev(const nb_params *p, const float *px,
 
 /* Number of compiled forward launch shapes, and a description of one:
  * block threads, targets per thread, LDS tile length, j-split count.
- * For a symmetric shape: 256 threads, particles per lane, super-tile length,
- * super-tiles per work item. */
+ * For a symmetric shape the fields name it: 256, particles per lane,
+ * super-tile length (256 times that), super-tiles per work item; for tile
+ * pairs the tile length (64 times that) and 1, or 2 for the shape that keeps
+ * rows of 128 particles at every n.  The workgroups that run have 256 or 512
+ * threads and 2, 4 or 8 targets per lane, by the shape and n. */
 int nb_forward_config_count(void);
 int nb_forward_config_info(int cfg, int *block, int *unroll, int *tile,
                            int *split);
